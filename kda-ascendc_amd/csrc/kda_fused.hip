@@ -8,13 +8,21 @@
 // for 1.4 GB of inputs and outputs).  Here one work-group per (sequence,
 // value head) keeps the records in LDS:
 //   * NP producer waves each form every NP-th chunk's record with stage 1's
-//     per-chunk code (k1_compute, kda_k1_chunk.h) straight into a ring of
-//     RING record slots in LDS, each with its own LDS scratch; each loads
-//     its next chunk's q, k and g rows into an LDS staging area while it
-//     works on the current one;
+//     per-chunk code (k1_compute, kda_k1_chunk.h) straight into their slot of
+//     a ring of RING record slots in LDS; each loads its next chunk's q, k
+//     and g rows into registers once this chunk's gates are done with, and v
+//     straight into the slot;
 //   * four compute waves each run the recurrence for two of the head's
 //     eight 16-column value tiles (wide_step, kda_k2w_step.h), reading the
 //     operands every tile shares from the slot.
+// Bound: the issue time of its vector and matrix instructions (an fp32 matrix
+// op holds the SIMD's vector unit for all of its 32 cycles, so the grams
+// alone are a sixth of it).  Twelve waves, three to a SIMD, so that two
+// others issue while one waits: with four producers at two waves per SIMD
+// the same work took as long as the waits it could not cover (B=16 T=2048
+// H=32: 490 us, and 450 us as it is now; 16 packed sequences in 8192 tokens,
+// 173 and 150 us).  The 168 registers of three waves per SIMD are the tight
+// side: a few spilled registers in the compute waves' loop cost 30 %.
 // The arithmetic is stage 1's and the wide stage 2's, so o and ht are bit
 // for bit those of the two-stage forward.
 //
@@ -43,22 +51,15 @@ namespace kda {
 namespace {
 
 constexpr int F_NCW = 4;  // compute waves, two value tiles each
-constexpr int F_NP = 4;   // producer waves
-constexpr int F_RING = 4; // record slots
+constexpr int F_NP = 8;   // producer waves
+constexpr int F_RING = 8; // record slots
 constexpr int F_THREADS = 64 * (F_NCW + F_NP);
 constexpr int SPIN_LIMIT = 1 << 22;
 static_assert(F_RING >= F_NP, "every producer can hold a slot");
 
-// A producer's staging area for the next chunk's q, k and g rows, which it
-// loads straight into LDS (direct buffer->LDS loads) while it works on the
-// current chunk: 16 rows of 256 bytes for q and k, of 256 (bf16) or 512
-// (fp32) bytes for g.
-constexpr int ST_Q = 0, ST_K = 4096, ST_G = 8192, STAGE_BYTES = 16384;
-
 // The work-group's LDS.
 __shared__ __attribute__((aligned(1024))) uint8_t f_ring[F_RING][FREC_BYTES];
-__shared__ __attribute__((aligned(1024))) uint8_t f_stage[F_NP][STAGE_BYTES];
-__shared__ __attribute__((aligned(16))) uint8_t f_scratch[F_NP][K1_SCRATCH];
+__shared__ __attribute__((aligned(16))) float f_L[F_RING][BT * BT];  // the solve's L
 __shared__ __attribute__((aligned(16))) float f_bias[DK];  // the head's dt_bias (zeros without it)
 __shared__ int f_full[F_RING];
 __shared__ int f_done[F_RING];
@@ -108,42 +109,43 @@ __device__ __forceinline__ void mark_lost(const Params& p, const SeqSpan& sp, in
 // The compute waves' side of the LDS flags (wide_step's hooks), and their
 // share of stage 1: u of their two tiles, formed from the raw v tiles,
 // bf16(A_inv) and beta the producers leave in u's place (FREC_*), with the
-// instructions stage 1 uses (form_u).  The producers pace the work-group;
-// this moves ~6 % of their issue work to the compute waves, which wait for
-// them most of the time.
-template <int S>
+// matrix op stage 1 uses (form_u).
 struct FlagHooks {
-    u32x2 v[2], a;  // raw v of the two tiles, bf16(A_inv) as the A operand
-    float beta;     // beta of this lane's row
-    __device__ __forceinline__ void ready(int c) { wait_ge(&f_full[S], c + 1); }
+    int s;          // the chunk's slot
+    i16x4 v[2], a;  // raw v of the two tiles in T order, bf16(A_inv) as the A operand
+    f32x4 beta;     // beta of rows 4*q4 .. +3
+    __device__ __forceinline__ void ready(int c) { wait_ge(&f_full[s], c + 1); }
+    __device__ __forceinline__ void read_kg(const uint8_t* slot, int lane, u32x4 (&kg)[4]) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const u32x2 k0 = __builtin_bit_cast(u32x2, get_T(slot + REC_KG, 2 * j, lane));
+            const u32x2 k1 = __builtin_bit_cast(u32x2, get_T(slot + REC_KG, 2 * j + 1, lane));
+            kg[j] = u32x4{k0.x, k0.y, k1.x, k1.y};
+        }
+    }
     __device__ __forceinline__ void read_u(const uint8_t* slot, int lane, int ut) {
-        v[0] = *reinterpret_cast<const u32x2*>(slot + REC_U + ut * 512 + lane * 8);
-        v[1] = *reinterpret_cast<const u32x2*>(slot + REC_U + (ut + 1) * 512 + lane * 8);
-        a = *reinterpret_cast<const u32x2*>(slot + FREC_A + lane * 8);
-        beta = *reinterpret_cast<const float*>(slot + FREC_BETA + 4 * (lane & 15));
+        // rows of 32 columns a load; the transposing read (get_T) of tile t's
+        // four-column pieces (pair_col)
+        typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+        const uint8_t* vs = slot + REC_U + (ut >> 1) * 1024 + (lane >> 2) * 64 + (lane & 3) * 16;
+        v[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)vs);
+        v[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vs + 8));
+        a = *reinterpret_cast<const i16x4*>(slot + FREC_A + lane * 8);
+        beta = *reinterpret_cast<const f32x4*>(slot + FREC_BETA + 16 * (lane >> 4));
     }
     __device__ __forceinline__ f32x4 u_start(int t) const {
-        const int lane = threadIdx.x & 63;
-        return unpack_u(form_u(v[t], beta, as_i16x4(a), eye_operand(lane)));
+        const u32x2 w = __builtin_bit_cast(u32x2, v[t]);
+        const u32x2 vb = pack4(lo_f(w.x) * beta[0], hi_f(w.x) * beta[1], lo_f(w.y) * beta[2], hi_f(w.y) * beta[3]);
+        return unpack_u(form_u(as_i16x4(vb), a));
     }
     __device__ __forceinline__ void consumed() {
         // the slot reads have completed before they are counted
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if ((threadIdx.x & 63) == 0)
-            __hip_atomic_fetch_add(&f_done[S], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_fetch_add(&f_done[s], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     __device__ __forceinline__ void end() {}
 };
-
-// Chunks c .. c + N - 1 (those below NT) from slot S on.
-template <int S, int N>
-__device__ __forceinline__ void fused_round(const WideCtx& cx, int c, f32x4 (&SA)[8], f32x4 (&SB)[8],
-                                            int ut) {
-    if (c >= cx.NT) return;
-    FlagHooks<S> hk;
-    wide_step(cx, c, SA, SB, f_ring[S], ut, hk);
-    if constexpr (N > 1) fused_round<(S + 1) % F_RING, N - 1>(cx, c + 1, SA, SB, ut);
-}
 
 // The LDS address of an LDS pointer (wave-uniform).
 __device__ __forceinline__ uint32_t lds_addr(const uint8_t* p) {
@@ -179,122 +181,112 @@ __device__ __forceinline__ void dma16(i32x4 rs, uint32_t lds, uint32_t voff) {
         : "=&s"(saved) : "s"(lds), "v"(voff), "s"(rs) : "memory");
 }
 
-// Staging layout: 16 rows of UNITS 16-byte units (16 for a bf16 row, 32
-// for an fp32 row); unit u of row r sits at position r * UNITS +
-// (u + r) % UNITS, so that the 16 lanes reading one unit column of the 16
-// rows hit 16 different bank groups.  One direct load moves 64 units (lane
-// l to position 64 i + l); rows past the sequence's end lie outside the
-// buffer descriptor's range, are not read, and are zeroed when read back.
-template <int UNITS>
-__device__ __forceinline__ void stage_issue(i32x4 rs, uint32_t dst, int lane, uint32_t row_stride) {
-#pragma unroll
-    for (int i = 0; i < UNITS / 4; ++i) {
-        const int pos = 64 * i + lane;
-        const int r = pos / UNITS;
-        const int u = (pos - r) & (UNITS - 1);
-        dma16(rs, dst + i * 1024, r * row_stride + u * 16);
-    }
-}
-
-// The direct loads of chunk c's q, k and g rows into the staging area at
-// LDS address st.
+// The q, k and g rows and beta of chunk c, in k1_load's layout.  Rows past
+// the sequence's end read its last row (in bounds; produce clears them).
 template <bool GB16>
-__device__ __forceinline__ void stage_chunk(const Params& p, int hv, int c, const SeqSpan& sp, uint32_t st,
-                                            int lane) {
-    const int h = hv / (p.HV / p.H);
-    const int nvalid = min(BT, sp.len - c * BT);
+__device__ __forceinline__ void load_chunk(const Params& p, int h, int hv, int c, const SeqSpan& sp, int lane,
+                                           K1In<GB16, false>& in) {
+    // a uniform base and a 32-bit offset per lane, so that the loads hold no
+    // 64-bit addresses in vector registers
+    const uint32_t r = min(lane & 15, sp.len - 1 - c * BT), q4 = lane >> 4;
     const int64_t tok = sp.tok0 + c * BT;
-    const uint32_t qs = (uint32_t)p.H * DK * 2, gs = (uint32_t)p.HV * DK * (GB16 ? 2 : 4);
-    const i32x4 rq = buffer_words(p.q + (tok * p.H + h) * DK, nvalid * qs);
-    const i32x4 rk = buffer_words(p.k + (tok * p.H + h) * DK, nvalid * qs);
-    const i32x4 rg = buffer_words(static_cast<const uint8_t*>(p.g) + (tok * p.HV + hv) * DK * (GB16 ? 2 : 4),
-                                  nvalid * gs);
-    stage_issue<16>(rq, st + ST_Q, lane, qs);
-    stage_issue<16>(rk, st + ST_K, lane, qs);
-    stage_issue<GB16 ? 16 : 32>(rg, st + ST_G, lane, gs);
-}
-
-// This lane's q, k and g values of the staged chunk, in k1_load's layout.
-template <bool FULL, bool GB16>
-__device__ __forceinline__ void stage_read(const uint8_t* st, int lane, bool valid, K1In<GB16, false>& in) {
-    const int r = lane & 15, q4 = lane >> 4;
+    const uint32_t qoff = r * (uint32_t)(p.H * DK * 2) + q4 * 8;
+    const uint32_t hvoff = r * (uint32_t)p.HV;
+    const uint8_t* qb = reinterpret_cast<const uint8_t*>(p.q + (tok * p.H + h) * DK);
+    const uint8_t* kb = reinterpret_cast<const uint8_t*>(p.k + (tok * p.H + h) * DK);
+    const uint8_t* gb = static_cast<const uint8_t*>(p.g) + (tok * p.HV + hv) * (DK * (GB16 ? 2 : 4));
+    const uint8_t* bb = static_cast<const uint8_t*>(p.beta) + (tok * p.HV + hv) * (p.beta_bf16 ? 2 : 4);
+    const uint32_t goff = hvoff * (DK * (GB16 ? 2 : 4)) + q4 * (GB16 ? 8 : 16);
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt) in.q.v[kt] = *reinterpret_cast<const u32x2*>(qb + 32 * kt + qoff);
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt) in.k.v[kt] = *reinterpret_cast<const u32x2*>(kb + 32 * kt + qoff);
 #pragma unroll
     for (int kt = 0; kt < 8; ++kt) {
-        const int b16 = (r * 16 + ((2 * kt + (q4 >> 1) + r) & 15)) * 16 + (q4 & 1) * 8;
-        in.q.v[kt] = *reinterpret_cast<const u32x2*>(st + ST_Q + b16);
-        in.k.v[kt] = *reinterpret_cast<const u32x2*>(st + ST_K + b16);
-        if constexpr (GB16) {
-            in.g16.v[kt] = *reinterpret_cast<const u32x2*>(st + ST_G + b16);
-        } else {
-            in.g32[kt] = *reinterpret_cast<const f32x4*>(st + ST_G + (r * 32 + ((4 * kt + q4 + r) & 31)) * 16);
-        }
-        if (!FULL && !valid) {
-            in.q.v[kt] = u32x2{0u, 0u};
-            in.k.v[kt] = u32x2{0u, 0u};
-            in.g16.v[kt] = u32x2{0u, 0u};
-            in.g32[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
+        if constexpr (GB16) in.g16.v[kt] = *reinterpret_cast<const u32x2*>(gb + 32 * kt + goff);
+        else in.g32[kt] = *reinterpret_cast<const f32x4*>(gb + 64 * kt + goff);
     }
+    if (p.beta_bf16) in.beta_bits = *reinterpret_cast<const uint16_t*>(bb + hvoff * 2);
+    else in.beta_bits = *reinterpret_cast<const uint32_t*>(bb + hvoff * 4);
 }
 
-// beta of this lane's row of chunk c (raw bits; 0 past the sequence's end).
-__device__ __forceinline__ uint32_t load_beta(const Params& p, int hv, int c, const SeqSpan& sp, int lane) {
-    const int r = lane & 15;
-    if (c * BT + r >= sp.len) return 0u;
-    const int64_t bi = (sp.tok0 + c * BT + r) * p.HV + hv;
-    return p.beta_bf16 ? static_cast<const uint16_t*>(p.beta)[bi] : static_cast<const uint32_t*>(p.beta)[bi];
-}
-
-// One chunk of a producer: its staged inputs to registers, v straight from
-// HBM (first used late in the chunk), the next chunk's staging and beta
-// issued, then stage 1's work into the ring slot.  `beta` holds this chunk's
-// beta on entry and the next chunk's on return.
+// A producer's side of its ring slot (k1_compute's hooks).
 template <bool FULL, bool GB16>
-__device__ __forceinline__ void produce(const Params& p, int hv, int c, int c_next, const SeqSpan& sp,
-                                        uint8_t* st, uint8_t* scr, float ea, uint32_t& beta, int lane) {
-    K1In<GB16, false> in;
-    const K1Row w = k1_row<FULL>(p, hv, c, sp);
-    // the staged rows of chunk c have landed (only direct loads are in flight)
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    stage_read<FULL, GB16>(st, lane, w.valid, in);
-    load_row(p.v + w.vrowoff, w.valid, w.colbase, in.v);
-    in.beta_bits = beta;
-    // the staging area is read before it is overwritten
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (c_next < sp.nt) {
-        stage_chunk<GB16>(p, hv, c_next, sp, lds_addr(st), lane);
-        beta = load_beta(p, hv, c_next, sp, lane);
+struct ProducerHooks {
+    const Params& p;
+    const SeqSpan& sp;
+    K1In<GB16, false>& in;
+    int h, hv, c, lane;
+    // Before the slot is written: its previous chunk has been read by every
+    // compute wave.  Then the chunk's v rows load straight into it.
+    __device__ __forceinline__ void slot() {
+        const int s = c % F_RING;
+        wait_ge(&f_done[s], F_NCW * (c / F_RING));
+        const int64_t row = ((sp.tok0 + c * BT) * p.HV + hv) * DK;
+        const uint32_t stride = (uint32_t)p.HV * DK * 2;
+        const i32x4 rs = buffer_words(p.v + row, min(BT, sp.len - c * BT) * stride);
+        // lane l of load j moves 16 bytes of row l / 4, columns 32*j + 8*(l % 4) .. +7
+        const uint32_t dst = lds_addr(f_ring[s] + REC_U);
+        const uint32_t off = (lane >> 2) * stride + (lane & 3) * 16;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dma16(rs, dst + j * 1024, off + j * 64);
     }
+    // q^, k^ and the gates are done with: the next chunk's rows load while
+    // the rest of this one is formed.  v has had the gram's time to land.
+    __device__ __forceinline__ void tail() {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if constexpr (!FULL) {
+            // v's rows past the sequence's end, which no load wrote
+            if ((lane >> 2) >= sp.len - c * BT) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    *reinterpret_cast<u32x4*>(f_ring[c % F_RING] + REC_U + j * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+            }
+        }
+        // (past the end: the last chunk again, so that the rows of this one
+        // are not held for it)
+        load_chunk<GB16>(p, h, hv, min(c + F_NP, sp.nt - 1), sp, lane, in);
+    }
+};
+
+// One chunk of a producer: stage 1's work on the rows in `in` into the ring
+// slot; on return `in` holds the next chunk's rows.
+template <bool FULL, bool GB16>
+__device__ __forceinline__ void produce(const Params& p, int h, int hv, int c, const SeqSpan& sp, float ea, int lane,
+                                        K1In<GB16, false>& in) {
     const int s = c % F_RING;
-    wait_ge(&f_done[s], F_NCW * (c / F_RING));
-    float* sL = reinterpret_cast<float*>(scr);
-    float* sX = reinterpret_cast<float*>(scr + K1_SCRATCH_L);
-    k1_compute<K1_FWD, FULL, GB16, true>(p, hv, c, sp, in, f_bias, ea, sL, sX, f_ring[s]);
+    if (!FULL && (lane & 15) >= sp.len - c * BT) {
+#pragma unroll
+        for (int kt = 0; kt < 8; ++kt) in.q.v[kt] = in.k.v[kt] = u32x2{0u, 0u};
+        in.beta_bits = 0u;
+    }
+    uint8_t* rec = f_ring[s];
+    // kb's tiles lie in w's bytes, kg's in kg's; the solve's columns where
+    // A_inv and beta go after it
+    const K1Scratch scr{f_L[s], reinterpret_cast<float*>(rec + FREC_A), rec + REC_W, rec + REC_KG};
+    const ProducerHooks<FULL, GB16> hk{p, sp, in, h, hv, c, lane};
+    k1_compute<K1_FWD, FULL, GB16, true>(p, hv, c, sp, in, f_bias, ea, scr, rec, hk);
     // the record's LDS writes have completed before the slot is marked full
+    // (v's rows had landed before tail() went on)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if (lane == 0) __hip_atomic_store(&f_full[s], c + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Producer wave pw: chunks pw, pw + NP, ... of the sequence, each into its
 // slot once the slot's previous chunk has been read by every compute wave.
-// The q, k and g rows of its next chunk load into its staging area while it
-// works on this one, so their HBM round trip overlaps that work.
 template <bool GB16>
 __device__ __forceinline__ void producer_wave(const Params& p, int pw, int hv, const SeqSpan& sp) {
     const int lane = threadIdx.x & 63;
-    uint8_t* st = f_stage[pw];
-    uint8_t* scr = f_scratch[pw];
     const float ea = k1_ea(p, hv);
     if (pw >= sp.nt) return;
-    stage_chunk<GB16>(p, hv, pw, sp, lds_addr(st), lane);
-    uint32_t beta = load_beta(p, hv, pw, sp, lane);
-    for (int c = pw; c < sp.nt; c += F_NP) {
-        if ((c + 1) * BT <= sp.len) {
-            produce<true, GB16>(p, hv, c, c + F_NP, sp, st, scr, ea, beta, lane);
-        } else {
-            produce<false, GB16>(p, hv, c, c + F_NP, sp, st, scr, ea, beta, lane);
-        }
-    }
+    const int h = __builtin_amdgcn_readfirstlane(hv / (p.HV / p.H));  // the q/k head of this value head
+    K1In<GB16, false> in;
+    load_chunk<GB16>(p, h, hv, pw, sp, lane, in);
+    // the full chunks, then the sequence's partial last one
+    const int nfull = sp.len / BT;
+    int c = pw;
+    for (; c < nfull; c += F_NP) produce<true, GB16>(p, h, hv, c, sp, ea, lane, in);
+    if (c < sp.nt) produce<false, GB16>(p, h, hv, c, sp, ea, lane, in);
 }
 
 // The (sequence or batch row, value head) of work-group wg.  A work-group
@@ -357,29 +349,33 @@ __global__ __launch_bounds__(F_THREADS) void fused_kernel(Params p) {
     __syncthreads();
 
     if (wave >= F_NCW) {
-        // The producers pace the work-group (B=16 T=2048 H=32: the compute
-        // waves' work alone takes 270 us, the producers' alone 900): on the
-        // SIMD a producer shares with a compute wave it issues first
-        // (649 -> 605 us).
+        // On the SIMD a producer shares with a compute wave it issues first:
+        // one long batch runs the same either way (B=16 T=2048 H=32: 450 us),
+        // 16 packed sequences in 8192 tokens in 150 us against 158 with the
+        // compute waves first or neither.
         __builtin_amdgcn_s_setprio(1);
         producer_wave<GB16>(p, wave - F_NCW, hv, sp);
         __builtin_amdgcn_endpgm();
     }
     const int ut = 2 * wave;                // this wave's first value tile
-    const int va = 16 * ut + (lane & 15);   // this lane's state row of it
+    // this lane's state rows of its two tiles
+    const int va = 16 * ut + pair_col(0, lane & 15), vb = 16 * ut + pair_col(1, lane & 15);
     f32x4 SA[8], SB[8];
     load_state(p, sbase, va, q4, SA);
-    load_state(p, sbase, va + 16, q4, SB);
+    load_state(p, sbase, vb, q4, SB);
     WideCtx cx;
     cx.scale = p.scale;
     cx.NT = sp.nt;
     cx.T = sp.len;
     cx.lane = lane;
     cx.q4 = q4;
-    cx.obase[0] = p.o + (sp.tok0 * p.HV + hv) * DK + 16 * ut + 4 * ((lane & 15) >> 2);
-    cx.obase[1] = cx.obase[0] + 16;
+    cx.obase = p.o + (sp.tok0 * p.HV + hv) * DK + 16 * ut + 8 * q4;
     cx.orow_stride = (int64_t)p.HV * DK;
-    for (int c = 0; c < cx.NT; c += F_RING) fused_round<0, F_RING>(cx, c, SA, SB, ut);
+    for (int c = 0; c < cx.NT; ++c) {
+        FlagHooks hk;
+        hk.s = c % F_RING;
+        wide_step(cx, c, SA, SB, f_ring[hk.s], ut, hk);
+    }
     // Every give-up is seen here by at least one compute wave: a producer
     // marks the work-group before it publishes the chunk it gave up on, and
     // this wave consumed every chunk; a compute wave sees its own.  The first
@@ -391,7 +387,7 @@ __global__ __launch_bounds__(F_THREADS) void fused_kernel(Params p) {
         mark_lost(p, sp, hv, ut, lane, SA, SB);
     }
     store_state(p, sbase, va, q4, SA);
-    store_state(p, sbase, va + 16, q4, SB);
+    store_state(p, sbase, vb, q4, SB);
     __builtin_amdgcn_endpgm();
 }
 

@@ -22,18 +22,20 @@ namespace kda {
 
 namespace {
 
-// Three waves per SIMD (at most 168 VGPRs; the compiler spills two 8-byte
-// values): each wave spends most of its life waiting on its loads, and a
-// third wave per SIMD hides more of that than the two that 172 VGPRs allow.
+// The forward's records: 122-129 VGPRs and 10 KiB of LDS a wave, so four waves
+// per SIMD (three with fp32 g and partial chunks).  A wave spends most of its
+// life waiting on memory, which sets the time (4.6 TB/s of a copy's 5.2);
+// held to three waves per SIMD B=2 T=4096 H=8 takes 100 against 96 us.
 //
 // K1M (the record modes, below) other than K1_FWD also writes the backward
 // record (kda_common.h) to p.ws_bwd: the same chunk quantities in the
 // operand orders of the reverse state chain, from one read of the inputs,
-// and the gram block to p.la.  Those modes run two waves per SIMD: they
-// hold more.
+// and the gram block to p.la.  Those modes hold more: K1_SAVE runs three
+// waves per SIMD, K1_BOTH two.
 // LDS of a work-group (one wave): k1_chunk's scratch.
 __shared__ __attribute__((aligned(16))) float s_L[BT * BT];
-__shared__ float s_X[BT * (BT + 1)];
+__shared__ float s_X[BT * BT];
+__shared__ __attribute__((aligned(16))) uint8_t s_kb[TILE_BYTES], s_kg[TILE_BYTES];
 
 // The (value head, chunk, sequence) of this work-group; false for a gap
 // slot (wave-uniform, before any barrier).  With cu_seqlens, slot x of
@@ -69,7 +71,7 @@ __attribute__((amdgpu_waves_per_eu(K1M != K1_FWD ? 2 : 3))) void k1_kernel(Param
     int hv, c;
     SeqSpan sp;
     if (!block_chunk(p, threadIdx.x, hv, c, sp)) return;
-    k1_chunk<K1M, ALL_FULL, GB16>(p, hv, c, sp, s_L, s_X, p.ws + (sp.rec0 + c) * REC_BYTES);
+    k1_chunk<K1M, ALL_FULL, GB16>(p, hv, c, sp, K1Scratch{s_L, s_X, s_kb, s_kg}, p.ws + (sp.rec0 + c) * REC_BYTES);
 }
 
 // The dO operand of each backward record that a training forward saved

@@ -22,7 +22,7 @@ struct Row32 {
 
 __device__ __forceinline__ float elem(const Row32& a, int p) {
     const uint32_t w = (p & 2) ? a.v[p >> 2].y : a.v[p >> 2].x;
-    return (p & 1) ? __builtin_bit_cast(float, w & 0xffff0000u) : __builtin_bit_cast(float, w << 16);
+    return (p & 1) ? hi_f(w) : lo_f(w);
 }
 
 __device__ __forceinline__ void load_row(const uint16_t* __restrict__ src, bool valid, int colbase,
@@ -59,26 +59,40 @@ __device__ __forceinline__ i16x4 tile_T(u32x2 f, i16x4 eye) {
     return as_i16x4(pack4(mfma_bf16_16x16x16(as_i16x4(f), eye, zero)));
 }
 
-// Tile vt of u = bf16(A @ bf16(v * beta)) (kernels.py:173-174) from the raw
-// v tile in F order (lane (r, q4) holding v[r][16*vt + 4*q4 + i]), the
-// lane's row's beta and bf16(A_inv) as the 16x16x16 A operand; it lands as
-// u[4*q4 + i][16*vt + r], the order stage 2 subtracts it in.  Stage 1 and
-// the fused forward's compute waves both form u with it.
-__device__ __forceinline__ u32x2 form_u(u32x2 v, float beta, i16x4 A_op, i16x4 eye) {
-    const float v0 = __builtin_bit_cast(float, v.x << 16);
-    const float v1 = __builtin_bit_cast(float, v.x & 0xffff0000u);
-    const float v2 = __builtin_bit_cast(float, v.y << 16);
-    const float v3 = __builtin_bit_cast(float, v.y & 0xffff0000u);
-    const i16x4 vbT = tile_T(pack4(v0 * beta, v1 * beta, v2 * beta, v3 * beta), eye);
+// The same transpose through LDS, for a whole 16x128 bf16 matrix: a tile
+// buffer holds [kt][row][16] (512 bytes a tile).  put_F writes tile kt from
+// F order, get_T reads it in T order with the transposing LDS read: in each
+// group of 16 lanes, lane n receives element n % 4 of lanes n / 4, 4 + n / 4,
+// 8 + n / 4, 12 + n / 4, so with lane l at byte 8 * l of the tile the group q4 holds
+// rows 4*q4 .. +3 and lane r takes their column r.  Both accesses cover 512
+// consecutive bytes: no bank conflicts.  Against tile_T a tile costs no
+// matrix op and no repacking (25 of the SIMD's cycles).
+constexpr int TILE_BYTES = BT * DK * 2;
+__device__ __forceinline__ void put_F(uint8_t* tiles, int kt, int lane, u32x2 f) {
+    *reinterpret_cast<u32x2*>(tiles + kt * 512 + (lane & 15) * 32 + (lane >> 4) * 8) = f;
+}
+__device__ __forceinline__ i16x4 get_T(const uint8_t* tiles, int kt, int lane) {
+    typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(tiles + kt * 512 + lane * 8));
+}
+
+// Tile vt of u = bf16(A @ bf16(v * beta)) (kernels.py:173-174) from
+// bf16(v * beta) in T order and bf16(A_inv) as the 16x16x16 A operand; it
+// lands as u[4*q4 + i][16*vt + r], the order stage 2 subtracts it in.  Stage
+// 1 and the fused forward's compute waves both form u with it.
+__device__ __forceinline__ u32x2 form_u(i16x4 vbT, i16x4 A_op) {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     return pack4(mfma_bf16_16x16x16(A_op, vbT, zero));
 }
 
-// LDS scratch of one wave's k1_chunk: L and the solve's columns (fp32), in
-// bytes.
-constexpr int K1_SCRATCH_L = BT * BT * 4;
-constexpr int K1_SCRATCH_X = BT * (BT + 1) * 4;
-constexpr int K1_SCRATCH = K1_SCRATCH_L + K1_SCRATCH_X;
+// LDS scratch of one wave's k1_compute: L and the solve's columns (fp32),
+// and the tile buffers of kb and kg.
+struct K1Scratch {
+    float* L;     // [16][16]
+    float* X;     // [16][16], column s at 16 * s, element t at t ^ s of it
+    uint8_t* kb;  // TILE_BYTES
+    uint8_t* kg;  // TILE_BYTES
+};
 
 // The wave's own LDS writes are complete before its next LDS read: the
 // scratch of k1_chunk belongs to one wave, so no work-group barrier is
@@ -95,12 +109,12 @@ enum K1Mode { K1_FWD = 0, K1_BOTH = 1, K1_SAVE = 2 };
 
 // The fused forward's ring slot (kda_fused.hip): the forward record with
 // u left to the compute waves, whose producers have the scarcer issue
-// slots.  In u's place the slot holds the chunk's raw v tiles in the
-// order u would take ([vt][lane][4] bf16, F order: lane (r, q4) holds
-// v[r][16*vt + 4*q4 + i]); then bf16(A_inv) as the 16x16x16 A operand
-// ([lane][4]) and beta per row as stage 1 applied it (fp32 [16]).  The
-// compute waves form u = bf16(A @ bf16(v * beta)) with the instructions
-// stage 1 uses (form_u), so u is the same bits.
+// slots.  In u's place the slot holds the chunk's raw v as tiles (put_F's
+// layout), then bf16(A_inv) as the 16x16x16 A operand ([lane][4]) and beta
+// per row as stage 1 applied it (fp32 [16]).  The compute waves form
+// u = bf16(A @ bf16(v * beta)) with the matrix op stage 1 uses (form_u), so u
+// is the same bits.  kg too stays as tiles, which the compute waves read in
+// T order (get_T).
 constexpr int FREC_A = REC_BYTES;
 constexpr int FREC_BETA = REC_BYTES + 512;
 constexpr int FREC_BYTES = REC_BYTES + 1024;
@@ -185,12 +199,22 @@ __device__ __forceinline__ float k1_ea(const Params& p, int hv) {
     return ea;
 }
 
+// Where a caller of k1_compute acts between its phases: `slot()` before the
+// first write to the record or the scratch, `tail()` once q^, k^ and the
+// gates are no longer needed.
+struct K1NoHooks {
+    __device__ __forceinline__ void slot() {}
+    __device__ __forceinline__ void tail() {}
+};
+
 // The work on one chunk's inputs: biasp the head's dt_bias (k1_bias, or a
-// copy of it), ea = k1_ea.
-template <int K1M, bool FULL, bool GB16, bool U_IN_SLOT = false>
+// copy of it), ea = k1_ea.  U_IN_SLOT: `rec` is a ring slot of the fused
+// forward (FREC_*); v is not touched here.
+template <int K1M, bool FULL, bool GB16, bool U_IN_SLOT = false, class Hooks = K1NoHooks>
 __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const SeqSpan& sp,
                                            const K1In<GB16, K1M == K1_BOTH>& in, const float* biasp,
-                                           float ea, float* sL, float* sX, uint8_t* rec) {
+                                           float ea, const K1Scratch& scr, uint8_t* rec,
+                                           Hooks hk = Hooks{}) {
     constexpr bool BOTH = K1M != K1_FWD;
     constexpr bool WITH_DO = K1M == K1_BOTH;
     const K1Row w = k1_row<FULL>(p, hv, c, sp);
@@ -206,9 +230,14 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
     const Row32& dop = in.dout;
     const Row32& gp = in.g16;
     const f32x4 (&gf)[8] = in.g32;
-    f32x4 bias[8];  // zeros without dt_bias (k1_bias), so s = g + bias either way
+    // zeros without dt_bias (k1_bias), so s = g + bias either way; loaded here
+    // from HBM, where it is used from LDS (the fused forward)
+    f32x4 bias[8];
+    auto load_bias = [&] {
 #pragma unroll
-    for (int kt = 0; kt < 8; ++kt) bias[kt] = *reinterpret_cast<const f32x4*>(biasp + 16 * kt + colbase);
+        for (int kt = 0; kt < 8; ++kt) bias[kt] = *reinterpret_cast<const f32x4*>(biasp + 16 * kt + colbase);
+    };
+    if constexpr (!U_IN_SLOT) load_bias();
     const uint32_t beta_bits = in.beta_bits;
     float G[32];
 #pragma unroll
@@ -223,16 +252,16 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
     if (p.use_l2norm) {
         float sq = 0.f, sk = 0.f;
 #pragma unroll
-        for (int j = 0; j < 32; ++j) {
-            sq = fmaf(elem(qp, j), elem(qp, j), sq);
-            sk = fmaf(elem(kp, j), elem(kp, j), sk);
+        for (int kt = 0; kt < 8; ++kt) {
+            sq = dot2(qp.v[kt].y, qp.v[kt].y, dot2(qp.v[kt].x, qp.v[kt].x, sq));
+            sk = dot2(kp.v[kt].y, kp.v[kt].y, dot2(kp.v[kt].x, kp.v[kt].x, sk));
         }
         sq += xor16(sq);
         sk += xor16(sk);
         sq += __shfl_xor(sq, 32);
         sk += __shfl_xor(sk, 32);
-        const float rq = 1.f / sqrtf(sq + L2_EPS);
-        const float rk = 1.f / sqrtf(sk + L2_EPS);
+        const float rq = __builtin_amdgcn_rsqf(sq + L2_EPS);
+        const float rk = __builtin_amdgcn_rsqf(sk + L2_EPS);
 #pragma unroll
         for (int kt = 0; kt < 8; ++kt) {
             qp.v[kt] = pack4(elem(qp, 4 * kt) * rq, elem(qp, 4 * kt + 1) * rq,
@@ -249,6 +278,7 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
     if (p.use_gate) {
         const float eal = ea * -1.4426950408889634f;
         const float lbr = p.lower_bound * RCP_LN2;
+        if constexpr (U_IN_SLOT) load_bias();
 #pragma unroll
         for (int kt = 0; kt < 8; ++kt) {
 #pragma unroll
@@ -283,18 +313,55 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
     };
     f32x4 acc_qk = {0.f, 0.f, 0.f, 0.f};
     f32x4 acc_kk = {0.f, 0.f, 0.f, 0.f};
+    // One pass over the columns forms everything that needs the gates: the
+    // grams' operands; kg = bf16(k^ * 2^(G_last - G)) (kernels.py:282-290) as
+    // the gram's k^ * 2^(G_mid - G) times row last's 2^(G_last - G_mid); kb =
+    // bf16(bf16(k^ * beta) * 2^G) (kernels.py:171); and qg = bf16(q^ * 2^G),
+    // the gated query stage 2 multiplies the state by (kernels.py:269).  kb
+    // and kg go to LDS tiles, to be read back in T order.  q^, k^ and G are
+    // unpacked and read once and die here, which leaves the rest of the chunk
+    // 122 registers where separate passes held 160.
+    hk.slot();
+    u32x2 kgF[8], qgp[8];
     bcast_mid([&](auto from_mid) {
+        bcast_last([&](auto from_last) {
 #pragma unroll
-        for (int j = 0; j < 32; ++j) {
-            const float gm = G[j] - from_mid(G[j]);
-            const float gq = valid ? fast_exp2(gm) : 0.f;
-            const float gk = valid ? fast_exp2(-gm) : 0.f;
-            const float qv = elem(qp, j), kv = elem(kp, j);
-            // A = Ks (rows s), B = Qs / Kq (columns t): lane (t, q4) receives
-            // Aqk[t][4*q4 + i] and Akk[t][4*q4 + i].
-            acc_qk = mfma_f32_16x16x4(kv * gk, qv * gq, acc_qk);
-            acc_kk = mfma_f32_16x16x4(kv * gk, kv * gq, acc_kk);
-        }
+            for (int kt = 0; kt < 8; ++kt) {
+                float kg[4], kb[4], qg[4], e[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int j = 4 * kt + i;
+                    const float gm = G[j] - from_mid(G[j]);
+                    const float gq = valid ? fast_exp2(gm) : 0.f;
+                    const float gk = valid ? fast_exp2(-gm) : 0.f;
+                    const float qv = elem(qp, j), kv = elem(kp, j);
+                    const float ks = kv * gk;
+                    // A = Ks (rows s), B = Qs / Kq (columns t): lane (t, q4)
+                    // receives Aqk[t][4*q4 + i] and Akk[t][4*q4 + i].
+                    acc_qk = mfma_f32_16x16x4(ks, qv * gq, acc_qk);
+                    acc_kk = mfma_f32_16x16x4(ks, kv * gq, acc_kk);
+                    kg[i] = ks * from_last(gq);
+                    e[i] = fast_exp2(G[j]);
+                    kb[i] = kv * beta;
+                    qg[i] = qv * e[i];
+                }
+                const u32x2 kbr = pack4(kb[0], kb[1], kb[2], kb[3]);
+                const u32x2 kbe = pack4(lo_f(kbr.x) * e[0], hi_f(kbr.x) * e[1],
+                                        lo_f(kbr.y) * e[2], hi_f(kbr.y) * e[3]);
+                put_F(scr.kb, kt, lane, kbe);
+                kgF[kt] = pack4(kg[0], kg[1], kg[2], kg[3]);
+                put_F(scr.kg, kt, lane, kgF[kt]);
+                // the state's decay 2^G_last (kernels.py:282-290): on the
+                // chunk's last row, 2^G is it
+                if (r == last)
+                    *reinterpret_cast<f32x4*>(rec + REC_DECAY + kt * 64 + q4 * 16) = f32x4{e[0], e[1], e[2], e[3]};
+                qgp[kt] = pack4(qg[0], qg[1], qg[2], qg[3]);
+                // (the backward's recompute produces no o and never reads qg)
+                if (K1M != K1_BOTH && (kt & 1))
+                    *reinterpret_cast<u32x4*>(rec + REC_QG + (kt >> 1) * 1024 + lane * 16) =
+                        u32x4{qgp[kt - 1].x, qgp[kt - 1].y, qgp[kt].x, qgp[kt].y};
+            }
+        });
     });
 
     // This chunk's record goes to `rec` with ordinary stores: in the
@@ -313,10 +380,12 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
     const u32x2 aqk_bf = pack4(aqk);
     *reinterpret_cast<u32x2*>(rec + REC_AQK + lane * 8) = aqk_bf;
 
+    hk.tail();
+
     // ---- (I + L)^-1 by forward substitution (kernels.py:157-167) ---------
     // Lane r solves column s = r: a[t] = A_inv[t][s], with a[s] = 1,
     // a[t < s] = 0 and a[t > s] = -sum_{j<t} L[t][j] a[j].
-    *reinterpret_cast<f32x4*>(sL + r * BT + 4 * q4) = L;
+    *reinterpret_cast<f32x4*>(scr.L + r * BT + 4 * q4) = L;
     wave_lds_fence();
     {
         float a[BT];
@@ -325,7 +394,7 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
             float acc = 0.f;
 #pragma unroll
             for (int j4 = 0; j4 < (t + 3) / 4; ++j4) {
-                const f32x4 lr = *reinterpret_cast<const f32x4*>(sL + t * BT + 4 * j4);
+                const f32x4 lr = *reinterpret_cast<const f32x4*>(scr.L + t * BT + 4 * j4);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     if (4 * j4 + i < t) acc = fmaf(-lr[i], a[4 * j4 + i], acc);
@@ -337,13 +406,13 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
         }
         if (q4 == 0) {
 #pragma unroll
-            for (int t = 0; t < BT; ++t) sX[r * (BT + 1) + t] = a[t];
+            for (int t = 0; t < BT; ++t) scr.X[r * BT + (t ^ r)] = a[t];
         }
     }
     wave_lds_fence();
     f32x4 ainv;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) ainv[i] = sX[(4 * q4 + i) * (BT + 1) + r];
+    for (int i = 0; i < 4; ++i) ainv[i] = scr.X[(4 * q4 + i) * BT + (r ^ (4 * q4 + i))];
     const u32x2 ainv_bf = pack4(ainv);  // A = bf16(A_inv), kernels.py:170
     if constexpr (BOTH) {
         // the gram and the inverse for the per-chunk gradients (kda_common.h)
@@ -355,6 +424,9 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
     const i16x4 A_neg = as_i16x4(ainv_bf ^ 0x80008000u);
     // the identity operand of the transposes through the matrix core (tile_T)
     const i16x4 eye = eye_operand(lane);
+    i16x4 kbT[8];
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt) kbT[kt] = get_T(scr.kb, kt, lane);
 
     if constexpr (BOTH) {
         // ---- backward record ---------------------------------------------
@@ -368,15 +440,11 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
         // order.
 #pragma unroll
         for (int kt = 0; kt < 8; ++kt) {
-            float kb[4], qs[4];
+            float qs[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float e = fast_exp2(G[4 * kt + i]);
-                kb[i] = round_bf(elem(kp, 4 * kt + i) * beta) * e;
-                qs[i] = p.scale * (elem(qp, 4 * kt + i) * e);
-            }
+            for (int i = 0; i < 4; ++i) qs[i] = p.scale * (elem(qp, 4 * kt + i) * fast_exp2(G[4 * kt + i]));
             const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-            const u32x2 wT = pack4(mfma_bf16_16x16x16(A_neg, tile_T(pack4(kb[0], kb[1], kb[2], kb[3]), eye), zero));
+            const u32x2 wT = pack4(mfma_bf16_16x16x16(A_neg, kbT[kt], zero));
             const u32x2 qv = __builtin_bit_cast(u32x2, tile_T(pack4(qs[0], qs[1], qs[2], qs[3]), eye));
             __builtin_nontemporal_store(u32x4{qv.x, qv.y, wT.x, wT.y},
                                         reinterpret_cast<u32x4*>(brec + BREC_UPD + kt * 1024 + lane * 16));
@@ -391,17 +459,12 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
         }
         // kg = bf16(k^ * 2^(G_last - G)) in F order (the A operand of
         // kg @ dh), and the decay 2^G_last.
-        u32x2 kgF[8];
         bcast_last([&](auto from_last) {
 #pragma unroll
             for (int kt = 0; kt < 8; ++kt) {
-                float kg[4], gl[4];
+                float gl[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    gl[i] = from_last(G[4 * kt + i]);
-                    kg[i] = elem(kp, 4 * kt + i) * fast_exp2(gl[i] - G[4 * kt + i]);
-                }
-                kgF[kt] = pack4(kg[0], kg[1], kg[2], kg[3]);
+                for (int i = 0; i < 4; ++i) gl[i] = from_last(G[4 * kt + i]);
                 if (r == 0)
                     __builtin_nontemporal_store(
                         f32x4{fast_exp2(gl[0]), fast_exp2(gl[1]), fast_exp2(gl[2]), fast_exp2(gl[3])},
@@ -415,21 +478,48 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
                 reinterpret_cast<u32x4*>(brec + BREC_KG + j * 1024 + lane * 16));
     }
 
+    // ---- w = A @ kb (kernels.py:171-172), computed transposed,
+    // w^T = kb^T @ A^T, so that tile kt lands as w[r][16*kt + 4*q4 + i]: F
+    // order, stage 2's operand.  The record holds -w (stage 2 forms
+    // u - w @ hc^T as one accumulation that starts at u): the product with
+    // -A, exact since negation commutes with the bf16 products, the fp32
+    // sums and the rounding.  (In the fused forward's slot kb's tiles lie in
+    // w's bytes: they have been read.)
+    u32x2 wpk[8];
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt) {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        wpk[kt] = pack4(mfma_bf16_16x16x16(kbT[kt], A_neg, zero));
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const u32x4 wj = {wpk[2 * j].x, wpk[2 * j].y, wpk[2 * j + 1].x, wpk[2 * j + 1].y};
+        *reinterpret_cast<u32x4*>(rec + REC_W + j * 1024 + lane * 16) = wj;
+    }
+
     // ---- u = A @ bf16(v * beta) (kernels.py:173-174) ----------------------
     // One 16x16x16 tile per 16 value columns; u lands as
-    // u[4*q4 + i][16*vt + r], the order stage 2 subtracts it in.  The
-    // transposes below go through the matrix core (tile_T).  In the fused
-    // forward's slot the operands go in u's place instead (FREC_*).
+    // u[4*q4 + i][16*vt + r], the order stage 2 subtracts it in.  In the
+    // fused forward's slot the operands go in u's place instead (FREC_*).
+    // kg goes out in T order (stage 2's A operand), or stays as tiles there.
     if constexpr (U_IN_SLOT) {
-#pragma unroll
-        for (int vt = 0; vt < 8; ++vt)
-            *reinterpret_cast<u32x2*>(rec + REC_U + vt * 512 + lane * 8) = vp.v[vt];
         *reinterpret_cast<u32x2*>(rec + FREC_A + lane * 8) = ainv_bf;
         if (q4 == 0) *reinterpret_cast<float*>(rec + FREC_BETA + 4 * r) = beta;
     } else {
 #pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const u32x2 k0 = __builtin_bit_cast(u32x2, get_T(scr.kg, 2 * j, lane));
+            const u32x2 k1 = __builtin_bit_cast(u32x2, get_T(scr.kg, 2 * j + 1, lane));
+            *reinterpret_cast<u32x4*>(rec + REC_KG + j * 1024 + lane * 16) = u32x4{k0.x, k0.y, k1.x, k1.y};
+        }
+#pragma unroll
+        for (int vt = 0; vt < 8; ++vt)
+            put_F(scr.kb, vt, lane, pack4(elem(vp, 4 * vt) * beta, elem(vp, 4 * vt + 1) * beta,
+                                          elem(vp, 4 * vt + 2) * beta, elem(vp, 4 * vt + 3) * beta));
+        wave_lds_fence();
+#pragma unroll
         for (int vt = 0; vt < 8; ++vt) {
-            const u32x2 ub = form_u(vp.v[vt], beta, A_op, eye);
+            const u32x2 ub = form_u(get_T(scr.kb, vt, lane), A_op);
             *reinterpret_cast<u32x2*>(rec + REC_U + vt * 512 + lane * 8) = ub;
             if (p.dbg_u) {
 #pragma unroll
@@ -445,71 +535,8 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
         }
     }
 
-    // ---- w = A @ bf16(bf16(k^ * beta) * 2^G) (kernels.py:171-172), and
-    // qg = bf16(q^ * 2^G), the gated query stage 2 multiplies the state by
-    // (kernels.py:269).  w is computed transposed, w^T = kb^T @ A^T, so that
-    // tile kt lands as w[r][16*kt + 4*q4 + i]: F order, stage 2's operand.
-    u32x2 qgp[8], kbF[8];
-#pragma unroll
-    for (int kt = 0; kt < 8; ++kt) {
-        float kb[4], qg[4], e[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            e[i] = fast_exp2(G[4 * kt + i]);
-            kb[i] = round_bf(elem(kp, 4 * kt + i) * beta) * e[i];
-            qg[i] = elem(qp, 4 * kt + i) * e[i];
-        }
-        kbF[kt] = pack4(kb[0], kb[1], kb[2], kb[3]);
-        qgp[kt] = pack4(qg[0], qg[1], qg[2], qg[3]);
-        // the state's decay 2^G_last (kernels.py:282-290): on the chunk's
-        // last row, 2^G is it
-        if (r == last)
-            *reinterpret_cast<f32x4*>(rec + REC_DECAY + kt * 64 + q4 * 16) = f32x4{e[0], e[1], e[2], e[3]};
-    }
-    // (the backward's recompute produces no o and never reads qg)
-    if constexpr (K1M != K1_BOTH) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const u32x4 qgj = {qgp[2 * j].x, qgp[2 * j].y, qgp[2 * j + 1].x, qgp[2 * j + 1].y};
-            *reinterpret_cast<u32x4*>(rec + REC_QG + j * 1024 + lane * 16) = qgj;
-        }
-    }
-    // The record holds -w (stage 2 forms u - w @ hc^T as one accumulation
-    // that starts at u): the product with -A, exact since negation commutes
-    // with the bf16 products, the fp32 sums and the rounding.
-    u32x2 wpk[8];
-#pragma unroll
-    for (int kt = 0; kt < 8; ++kt) {
-        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-        wpk[kt] = pack4(mfma_bf16_16x16x16(tile_T(kbF[kt], eye), A_neg, zero));
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const u32x4 wj = {wpk[2 * j].x, wpk[2 * j].y, wpk[2 * j + 1].x, wpk[2 * j + 1].y};
-        *reinterpret_cast<u32x4*>(rec + REC_W + j * 1024 + lane * 16) = wj;
-    }
-
-    // ---- kg = bf16(k^ * 2^(G_last - G)) (kernels.py:282-290), stored in T
-    // order (stage 2's A operand).
-    bcast_last([&](auto from_last) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            u32x2 kgT[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int kt = 2 * j + h;
-                float kg[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    kg[i] = elem(kp, 4 * kt + i) * fast_exp2(from_last(G[4 * kt + i]) - G[4 * kt + i]);
-                kgT[h] = __builtin_bit_cast(u32x2, tile_T(pack4(kg[0], kg[1], kg[2], kg[3]), eye));
-            }
-            *reinterpret_cast<u32x4*>(rec + REC_KG + j * 1024 + lane * 16) =
-                u32x4{kgT[0].x, kgT[0].y, kgT[1].x, kgT[1].y};
-        }
-    });
-
     // ---- optional reference-layout intermediates (kernels.py:125,153,178-184)
+    if constexpr (U_IN_SLOT) return;
     if (p.dbg_w && valid) {
         const int64_t bt16 = (tok * HV + hv) * BT + 4 * q4;
         *reinterpret_cast<u32x2*>(p.dbg_Aqk + bt16) = aqk_bf;
@@ -529,12 +556,12 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
 // GB16: g is bf16 (else fp32).
 template <int K1M, bool FULL, bool GB16>
 __device__ __forceinline__ void k1_chunk(const Params& p, int hv, int c, const SeqSpan& sp,
-                                         float* sL, float* sX, uint8_t* rec) {
+                                         const K1Scratch& scr, uint8_t* rec) {
     K1In<GB16, K1M == K1_BOTH> in;
     k1_load<K1M, FULL, GB16>(p, hv, c, sp, in);
     const float* biasp = k1_bias(p, hv);
     const float ea = k1_ea(p, hv);
-    k1_compute<K1M, FULL, GB16>(p, hv, c, sp, in, biasp, ea, sL, sX, rec);
+    k1_compute<K1M, FULL, GB16>(p, hv, c, sp, in, biasp, ea, scr, rec);
 }
 
 }  // namespace

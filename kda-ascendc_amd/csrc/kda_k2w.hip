@@ -140,13 +140,15 @@ __global__ __launch_bounds__((WideGeom<TPW, TW>::THREADS)) void k2w_kernel(Param
         const int ut = TW * wave;              // first of this wave's tiles in the slice
         const int vt = slice * TPW + ut;       // its value tile
         const int q4 = lane >> 4;
-        const int va = 16 * vt + (lane & 15);  // this lane's state row (V index) of tile A
+        // this lane's state rows (V index) of tiles A and B
+        const int va = 16 * vt + (TW == 2 ? pair_col(0, lane & 15) : lane & 15);
+        const int vb = 16 * vt + pair_col(1, lane & 15);
         f32x4 SA[8], SB[8];
         load_state(p, sbase, va, q4, SA);
-        if (TW == 2) load_state(p, sbase, va + 16, q4, SB);
+        if (TW == 2) load_state(p, sbase, vb, q4, SB);
         if (sp.nt == 0) {  // an empty sequence: the final state is the initial state
             store_state(p, sbase, va, q4, SA);
-            if (TW == 2) store_state(p, sbase, va + 16, q4, SB);
+            if (TW == 2) store_state(p, sbase, vb, q4, SB);
             __builtin_amdgcn_endpgm();
         }
         WideCtx cx;
@@ -155,14 +157,14 @@ __global__ __launch_bounds__((WideGeom<TPW, TW>::THREADS)) void k2w_kernel(Param
         cx.T = sp.len;
         cx.lane = lane;
         cx.q4 = q4;
-        const int col = 4 * ((lane & 15) >> 2);
-        cx.obase[0] = p.o + (sp.tok0 * p.HV + hv) * DK + 16 * vt + col;
-        cx.obase[1] = cx.obase[0] + 16;
+        // the first column of o this lane stores (8 with two tiles, 4 with one)
+        const int col = TW == 2 ? 8 * q4 : 4 * ((lane & 15) >> 2);
+        cx.obase = p.o + (sp.tok0 * p.HV + hv) * DK + 16 * vt + col;
         cx.orow_stride = (int64_t)p.HV * DK;
         chunk_barrier();  // chunk 0 is in the ring
         for (int c = 0; c < cx.NT; c += G::RING) wide_round<TPW, TW, 0, G::RING>(cx, c, SA, SB, ring, ut);
         store_state(p, sbase, va, q4, SA);
-        if (TW == 2) store_state(p, sbase, va + 16, q4, SB);
+        if (TW == 2) store_state(p, sbase, vb, q4, SB);
         __builtin_amdgcn_endpgm();
     }
     // copy wave

@@ -10,24 +10,24 @@
 namespace kda {
 namespace {
 
-// The operands a compute wave reads for one chunk.
+// The operands a compute wave reads for one chunk: those of v_new and o,
+// then those of the state update.
 struct WideOps {
     u32x4 w[4];   // -w, 16x16x32 A operands (k-tile pairs)
-    u32x4 qg[4];  // qg, likewise
+    u32x4 qg[4];  // qg, likewise (B operands)
+    u32x2 aqk;    // Aqk, 16x16x16 B operand
+};
+struct WideUpd {
     u32x4 kg[4];  // kg, 16x16x16 A operands of the update (two k-tiles each)
-    u32x2 aqk;    // Aqk, 16x16x16 A operand
-    f32x2 dc;     // 2^G_last for the decay broadcast
+    f32x4 dc[8];  // 2^G_last of this lane's k rows: [kt][i] of k = 16*kt + 4*q4 + i
 };
 
-__device__ __forceinline__ void read_wide_ops(const uint8_t* slot, int lane, int ut, WideOps& op) {
+__device__ __forceinline__ void read_wide_ops(const uint8_t* slot, int lane, WideOps& op) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        op.w[j] = *reinterpret_cast<const u32x4*>(slot + REC_W + j * 1024 + lane * 16);
-        op.qg[j] = *reinterpret_cast<const u32x4*>(slot + REC_QG + j * 1024 + lane * 16);
-        op.kg[j] = *reinterpret_cast<const u32x4*>(slot + REC_KG + j * 1024 + lane * 16);
-    }
+    for (int j = 0; j < 4; ++j) op.w[j] = *reinterpret_cast<const u32x4*>(slot + REC_W + j * 1024 + lane * 16);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) op.qg[j] = *reinterpret_cast<const u32x4*>(slot + REC_QG + j * 1024 + lane * 16);
     op.aqk = *reinterpret_cast<const u32x2*>(slot + REC_AQK + lane * 8);
-    op.dc = *reinterpret_cast<const f32x2*>(slot + decay_offset(lane));
 }
 
 __device__ __forceinline__ f32x4 unpack_u(u32x2 u) {
@@ -43,19 +43,26 @@ __device__ __forceinline__ u32x4 pack_hc(const f32x4 (&St)[8], int j) {
 }
 
 // k-tile KT of both tiles' state update: S = S * 2^G_last + kg^T v_new (the
-// decay a VALU product on the accumulator input, as kda_k2.hip forms it).
+// decay a VALU product on the accumulator input, as kda_k2.hip forms it; the
+// factors of both tiles' products come from registers, which a plain product
+// reads at twice the rate of a DPP broadcast).
 template <int KT>
-__device__ __forceinline__ void wide_update(f32x4 (&SA)[8], f32x4 (&SB)[8], const WideOps& op,
+__device__ __forceinline__ void wide_update(f32x4 (&SA)[8], f32x4 (&SB)[8], const WideUpd& op,
                                             u32x2 vna, u32x2 vnb) {
     const u32x4 kg = op.kg[KT >> 1];
     const i16x4 a = as_i16x4((KT & 1) ? u32x2{kg.z, kg.w} : u32x2{kg.x, kg.y});
-    SA[KT] = mfma_bf16_16x16x16(a, as_i16x4(vna), decay_tile<KT>(SA[KT], op.dc));
-    SB[KT] = mfma_bf16_16x16x16(a, as_i16x4(vnb), decay_tile<KT>(SB[KT], op.dc));
+    SA[KT] = mfma_bf16_16x16x16(a, as_i16x4(vna), SA[KT] * op.dc[KT]);
+    SB[KT] = mfma_bf16_16x16x16(a, as_i16x4(vnb), SB[KT] * op.dc[KT]);
 }
+
+// The value column of lane x of tile t (0, 1) of a wave's 32 columns: the two
+// tiles interleave in fours, so that the o a lane receives (columns 4*q4 ..
+// +3 of both tiles, formed transposed) is 8 consecutive columns of its row.
+__device__ __forceinline__ int pair_col(int t, int x) { return 8 * (x >> 2) + 4 * t + (x & 3); }
 
 // Constants of a compute wave.
 struct WideCtx {
-    uint16_t* obase[2];   // o of the sequence's first token, this lane's 4 columns of each tile
+    uint16_t* obase;      // o of the sequence's first token, the first column this lane stores
     int64_t orow_stride;  // elements between consecutive tokens of o
     float scale;
     int NT, T, lane, q4;
@@ -63,7 +70,7 @@ struct WideCtx {
 
 // How the waves of a work-group meet around one chunk of a compute wave:
 // `ready(c)` before the wave reads chunk c's operands from their ring slot,
-// `consumed()` once those reads are issued, `end()` after the chunk; and
+// `consumed()` once its last reads are issued, `end()` after the chunk; and
 // where u comes from: `read_u` with the slot reads, `u_start(t)` for tile
 // t's accumulator start after them.  kda_k2w.hip: one barrier per chunk,
 // u as stage 1 stored it (BarrierHooks); kda_fused.hip: LDS flags between
@@ -72,9 +79,18 @@ struct WideCtx {
 struct BarrierHooks {
     u32x2 u[2];  // u of the two tiles (bf16 pairs)
     __device__ __forceinline__ void ready(int) {}
+    __device__ __forceinline__ void read_kg(const uint8_t* slot, int lane, u32x4 (&kg)[4]) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) kg[j] = *reinterpret_cast<const u32x4*>(slot + REC_KG + j * 1024 + lane * 16);
+    }
     __device__ __forceinline__ void read_u(const uint8_t* slot, int lane, int ut) {
-        u[0] = *reinterpret_cast<const u32x2*>(slot + REC_SHARED + ut * 512 + lane * 8);
-        u[1] = *reinterpret_cast<const u32x2*>(slot + REC_SHARED + (ut + 1) * 512 + lane * 8);
+        // u of column 16*ut + pair_col(t, x): tile ut + col / 16, its lane col % 16
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int col = pair_col(t, lane & 15);
+            u[t] = *reinterpret_cast<const u32x2*>(slot + REC_SHARED + (ut + (col >> 4)) * 512 +
+                                                   (lane >> 4) * 128 + (col & 15) * 8);
+        }
     }
     __device__ __forceinline__ void consumed() {}
     __device__ __forceinline__ f32x4 u_start(int t) const { return unpack_u(u[t]); }
@@ -82,15 +98,15 @@ struct BarrierHooks {
 };
 
 // One chunk of a compute wave: both tiles' v_new, o and state update, with
-// chunk c's operands read from its ring slot at the start.  The reads are
-// covered by the packing of hc, which needs only the state; one operand set
-// is live at a time.
+// chunk c's operands read from its ring slot: those of v_new and o at the
+// start, covered by the packing of hc, which needs only the state; those of
+// the update behind the first products.
 template <class Hooks>
 __device__ __forceinline__ void wide_step(const WideCtx& cx, int c, f32x4 (&SA)[8], f32x4 (&SB)[8],
                                           const uint8_t* slot, int ut, Hooks& hk) {
     hk.ready(c);
     WideOps cur;
-    read_wide_ops(slot, cx.lane, ut, cur);
+    read_wide_ops(slot, cx.lane, cur);
     hk.read_u(slot, cx.lane, ut);
     u32x4 ha[4], hb[4];
 #pragma unroll
@@ -98,7 +114,6 @@ __device__ __forceinline__ void wide_step(const WideCtx& cx, int c, f32x4 (&SA)[
         ha[j] = pack_hc(SA, j);
         hb[j] = pack_hc(SB, j);
     }
-    hk.consumed();
     // v_new = u - w @ hc^T: one accumulation chain per tile, from u
     f32x4 va = hk.u_start(0);
     f32x4 vb = hk.u_start(1);
@@ -107,43 +122,48 @@ __device__ __forceinline__ void wide_step(const WideCtx& cx, int c, f32x4 (&SA)[
         va = mfma_bf16_16x16x32(as_bf16x8(cur.w[j]), as_bf16x8(ha[j]), va);
         vb = mfma_bf16_16x16x32(as_bf16x8(cur.w[j]), as_bf16x8(hb[j]), vb);
     }
-    // o = scale * qg @ hc^T + Aqk @ v_new
+    // o = scale * qg @ hc^T + Aqk @ v_new, formed transposed (the operands
+    // of each product swapped: the same sums), so that lane (t, q4) receives
+    // columns 4*q4 .. +3 of both tiles in row t: 16 consecutive bytes
+    // (pair_col)
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 oa = zero, ob = zero;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        oa = mfma_bf16_16x16x32(as_bf16x8(cur.qg[j]), as_bf16x8(ha[j]), oa);
-        ob = mfma_bf16_16x16x32(as_bf16x8(cur.qg[j]), as_bf16x8(hb[j]), ob);
+        oa = mfma_bf16_16x16x32(as_bf16x8(ha[j]), as_bf16x8(cur.qg[j]), oa);
+        ob = mfma_bf16_16x16x32(as_bf16x8(hb[j]), as_bf16x8(cur.qg[j]), ob);
     }
+    // The update's operands are read only now: with those above they would
+    // not fit the 168 registers of three waves per SIMD.
+    __builtin_amdgcn_sched_barrier(0);
+    WideUpd upd;
+    hk.read_kg(slot, cx.lane, upd.kg);
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt)
+        upd.dc[kt] = *reinterpret_cast<const f32x4*>(slot + REC_DECAY + kt * 64 + cx.q4 * 16);
+    hk.consumed();
     const u32x2 vna = {pack2(va[0], va[1]), pack2(va[2], va[3])};
     const u32x2 vnb = {pack2(vb[0], vb[1]), pack2(vb[2], vb[3])};
     oa = oa * cx.scale;
     ob = ob * cx.scale;
-    oa = mfma_bf16_16x16x16(as_i16x4(cur.aqk), as_i16x4(vna), oa);
-    ob = mfma_bf16_16x16x16(as_i16x4(cur.aqk), as_i16x4(vnb), ob);
+    oa = mfma_bf16_16x16x16(as_i16x4(vna), as_i16x4(cur.aqk), oa);
+    ob = mfma_bf16_16x16x16(as_i16x4(vnb), as_i16x4(cur.aqk), ob);
     // state update: S = S * 2^G_last + kg^T v_new, tile by tile
-    wide_update<0>(SA, SB, cur, vna, vnb);
-    wide_update<1>(SA, SB, cur, vna, vnb);
-    wide_update<2>(SA, SB, cur, vna, vnb);
-    wide_update<3>(SA, SB, cur, vna, vnb);
-    wide_update<4>(SA, SB, cur, vna, vnb);
-    wide_update<5>(SA, SB, cur, vna, vnb);
-    wide_update<6>(SA, SB, cur, vna, vnb);
-    wide_update<7>(SA, SB, cur, vna, vnb);
-    // Lane (x, q4) holds o rows 4*q4 .. +3 of column x; after the quad
-    // transpose it holds row 4*q4 + x%4, columns 4*(x/4) .. +3.
-    const int j4 = cx.lane & 3;
-    const u32x2 ota = quad_transpose(pack2(oa[0], oa[1]), pack2(oa[2], oa[3]), j4);
-    const u32x2 otb = quad_transpose(pack2(ob[0], ob[1]), pack2(ob[2], ob[3]), j4);
-    // Ordinary stores: the 8-byte pieces of one 256-byte row of o come from
+    wide_update<0>(SA, SB, upd, vna, vnb);
+    wide_update<1>(SA, SB, upd, vna, vnb);
+    wide_update<2>(SA, SB, upd, vna, vnb);
+    wide_update<3>(SA, SB, upd, vna, vnb);
+    wide_update<4>(SA, SB, upd, vna, vnb);
+    wide_update<5>(SA, SB, upd, vna, vnb);
+    wide_update<6>(SA, SB, upd, vna, vnb);
+    wide_update<7>(SA, SB, upd, vna, vnb);
+    // Ordinary stores: the pieces of one 256-byte row of o come from
     // different waves, and merge in L2 (non-temporal stores of the same
     // pieces made stage 2 ~10% slower at B=1 T=8192 H=96).
-    const int t = c * BT + 4 * cx.q4 + j4;
-    if (t < cx.T) {
-        const int64_t off = (int64_t)t * cx.orow_stride;
-        *reinterpret_cast<u32x2*>(cx.obase[0] + off) = ota;
-        *reinterpret_cast<u32x2*>(cx.obase[1] + off) = otb;
-    }
+    const int t = c * BT + (cx.lane & 15);
+    if (t < cx.T)
+        *reinterpret_cast<u32x4*>(cx.obase + (int64_t)t * cx.orow_stride) =
+            u32x4{pack2(oa[0], oa[1]), pack2(oa[2], oa[3]), pack2(ob[0], ob[1]), pack2(ob[2], ob[3])};
     hk.end();
 }
 
@@ -195,7 +215,7 @@ __device__ __forceinline__ void wide1_step(const WideCtx& cx, int c, f32x4 (&S)[
     const int j4 = cx.lane & 3;
     const u32x2 ot = quad_transpose(pack2(o[0], o[1]), pack2(o[2], o[3]), j4);
     const int t = c * BT + 4 * cx.q4 + j4;
-    if (t < cx.T) *reinterpret_cast<u32x2*>(cx.obase[0] + (int64_t)t * cx.orow_stride) = ot;
+    if (t < cx.T) *reinterpret_cast<u32x2*>(cx.obase + (int64_t)t * cx.orow_stride) = ot;
     chunk_barrier();
 }
 
