@@ -96,7 +96,7 @@ __device__ __forceinline__ void lds_get8(const float* src, float (&x)[8]) {
 // One value head's row data of this thread (row i, columns c0 .. c0+7):
 // g is the gate's argument g + dt_bias with the in-kernel gate, else g.
 struct HvRow {
-    float v[8], g[8], dvn[8];
+    float g[8], dvn[8];
     float beta, alog;
 };
 
@@ -127,20 +127,24 @@ struct HdhOps {
 };
 
 // GROUP: grouped value heads (HV > H), the value heads of a q/k head in a
-// loop.  Without it the body runs once, and the compiler keeps nothing live
-// across iterations (hoisted addresses and row values would otherwise hold
-// registers through the whole body).  FULL: a fixed-length batch with T a
+// loop.  Without it the body runs once.  Either way two work-groups share a
+// CU (76 KiB of LDS and at most 256 VGPRs each): a group's loop keeps what it
+// could hoist (coordinates, addresses, q^, k^) out of registers, and loads
+// h and dh' at an iteration's start but the rows of dO, dv_new and v_new only
+// before their products.  One work-group per CU took it 221 us at 4000 packed
+// tokens, H = 8, HV = 16, two 149.  FULL: a fixed-length batch with T a
 // multiple of 16, so every row of every chunk is a token (no row-validity
 // selects).
 template <bool GROUP, bool FULL>
-__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 2))) void bwd_chunk_kernel(Params p) {
+__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(2))) void bwd_chunk_kernel(Params p) {
     __shared__ ChunkSmem sm;
-    const int t = threadIdx.x;
-    const int lane = t & 63, w = t >> 6;
-    const int x = lane & 15, q4 = lane >> 4;  // matrix-op lane coordinates
-    const int i = t >> 4;          // row (and row of the 16x16 mapping)
-    const int cb = t & 15;         // column of the 16x16 mapping
-    const int c0 = 8 * cb;         // first of this thread's 8 columns
+    int t = threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    int lane = t & 63;
+    int x = lane & 15, q4 = lane >> 4;  // matrix-op lane coordinates
+    int i = t >> 4;          // row (and row of the 16x16 mapping)
+    int cb = t & 15;         // column of the 16x16 mapping
+    int c0 = 8 * cb;         // first of this thread's 8 columns
     const int H = p.H, HV = p.HV, rep = HV / H;
     const bool gate_grads = p.use_gate && p.tr_part;
 
@@ -166,47 +170,47 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
         h = bq - seq * H;
     }
     const SeqSpan sq = seq_span(p, seq * HV + h * rep);
-    const int nvalid = min(BT, sq.len - c * BT);
-    const int mid = min(BT / 2, nvalid - 1), last = nvalid - 1;
+    int nvalid = FULL ? BT : __builtin_amdgcn_readfirstlane(min(BT, sq.len - c * BT));
+    int mid = min(BT / 2, nvalid - 1), last = nvalid - 1;
     const bool valid = FULL || i < nvalid;
-    const int64_t tok = sq.tok0 + c * BT + i;
+    const int64_t tok0 = sq.tok0 + c * BT;  // the chunk's first token
 
     // Every load of a value head is issued before the first wait.  Rows
     // past the chunk's last token read that token's row (in bounds) and are
     // zeroed where they are used; absent operands read kZeroCols.
-    const int64_t tokc = sq.tok0 + c * BT + (valid ? i : nvalid - 1);
+    auto rowc = [&] { return (uint32_t)(valid ? i : nvalid - 1); };
     const bool has_bias = p.use_gate && p.dt_bias;
     auto load_hv = [&](int hv, HvRaw& r) {
         const SeqSpan sp = seq_span(p, seq * HV + hv);
         const int64_t rec = sp.rec0 + c;
-        const int64_t vrow = (tokc * HV + hv) * DK;
+        // uniform bases and 32-bit lane offsets (load_ops)
+        const uint32_t ho = rowc() * (uint32_t)HV, vo = ho * DK + c0;
+        const int64_t bi = tok0 * HV + hv;
         // (the row loads last: an address formed after a load may take that
         // load's destination registers and wait for it)
-        const int64_t bi = tokc * HV + hv;
-        if (p.beta_bf16) r.beta = static_cast<const uint16_t*>(p.beta)[bi];
-        else r.beta = static_cast<const uint32_t*>(p.beta)[bi];
+        if (p.beta_bf16) r.beta = (static_cast<const uint16_t*>(p.beta) + bi)[ho];
+        else r.beta = (static_cast<const uint32_t*>(p.beta) + bi)[ho];
         r.alog = *(p.use_gate ? p.A_log + hv : kZeroCols);
         const float* laf = reinterpret_cast<const float*>(p.la + rec * p.la_stride);
-        r.lraw = laf[LA_LRAW / 4 + (i + 16 * (cb >> 2)) * 4 + (cb & 3)];
-        r.ainv = laf[LA_AINV / 4 + (i + 16 * (cb >> 2)) * 4 + (cb & 3)];
+        const uint32_t lo = (i + 16 * (cb >> 2)) * 4 + (cb & 3);
+        r.lraw = (laf + LA_LRAW / 4)[lo];
+        r.ainv = (laf + LA_AINV / 4)[lo];
         const float* biasp = has_bias ? p.dt_bias + hv * DK : kZeroCols;
-        r.bias[0] = *reinterpret_cast<const f32x4*>(biasp + c0);
-        r.bias[1] = *reinterpret_cast<const f32x4*>(biasp + c0 + 4);
-        r.dvn = *reinterpret_cast<const u32x4*>(p.tr_dvn + rec * TR_VN_ELEMS + (cb >> 1) * TR_VN_TILE +
-                                                i * 16 + 8 * (cb & 1));
-        r.v = *reinterpret_cast<const u32x4*>(p.v + vrow + c0);
+        r.bias[0] = *reinterpret_cast<const f32x4*>(biasp + (uint32_t)c0);
+        r.bias[1] = *reinterpret_cast<const f32x4*>(biasp + 4 + (uint32_t)c0);
+        r.dvn = *reinterpret_cast<const u32x4*>(p.tr_dvn + rec * TR_VN_ELEMS +
+                                                (uint32_t)((cb >> 1) * TR_VN_TILE + i * 16 + 8 * (cb & 1)));
+        r.v = *reinterpret_cast<const u32x4*>(p.v + bi * DK + vo);
         // bf16: 16 bytes (read twice); fp32: 32 bytes
-        const uint32_t* gsrc = p.g_bf16
-            ? reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(p.g) + vrow + c0)
-            : reinterpret_cast<const uint32_t*>(static_cast<const float*>(p.g) + vrow + c0);
-        r.g[0] = *reinterpret_cast<const u32x4*>(gsrc);
-        r.g[1] = *reinterpret_cast<const u32x4*>(gsrc + (p.g_bf16 ? 0 : 4));
+        const uint8_t* gb = static_cast<const uint8_t*>(p.g) + bi * DK * (p.g_bf16 ? 2 : 4);
+        const uint32_t go = vo * (p.g_bf16 ? 2 : 4);
+        r.g[0] = *reinterpret_cast<const u32x4*>(gb + go);
+        r.g[1] = *reinterpret_cast<const u32x4*>(gb + (p.g_bf16 ? 0 : 16) + go);
     };
     // g is the gate's argument g + dt_bias with the in-kernel gate; rows
     // past the last token hold v = dv_new = beta = 0 and g = dt_bias.
     auto decode_hv = [&](const HvRaw& r, HvRow& o) {
-        float v[8], dv[8], g[8];
-        unpack8(r.v, v);
+        float dv[8], g[8];
         unpack8(r.dvn, dv);
         if (p.g_bf16) {
             unpack8(r.g[0], g);
@@ -222,7 +226,6 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            o.v[j] = valid ? v[j] : 0.f;
             o.dvn[j] = valid ? dv[j] : 0.f;
             const float gv = valid ? g[j] : 0.f;
             o.g[j] = has_bias ? gv + r.bias[j >> 2][j & 3] : gv;
@@ -231,29 +234,41 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
         o.beta = valid ? b : 0.f;
         o.alog = r.alog;
     };
-    auto load_ops = [&](int hv, HdhOps& o) {
+    // The row's v, unpacked where it is used (packed it holds half the
+    // registers in between).
+    auto row_v = [&](u32x4& packed, float (&v)[8]) {
+        if constexpr (GROUP) asm volatile("" : "+v"(packed));
+        unpack8(packed, v);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = valid ? v[j] : 0.f;
+    };
+    // (rows: dO, dv_new, v_new; tiles: h, dh')
+    auto load_ops = [&](int hv, HdhOps& o, bool rows, bool tiles) {
         const int64_t rec = seq_span(p, seq * HV + hv).rec0 + c;
+        // Uniform bases and one 32-bit lane offset each, so that the loads
+        // hold no 64-bit addresses in vector registers.  Blocked layouts:
+        // v = 32*jv + 8*q4 + e lies in value tile 2*jv + q4/2 at column
+        // 8*(q4%2) + e
         const uint16_t* hrec = p.tr_h + rec * TR_H_ELEMS;
         const uint16_t* dhrec = p.tr_dh + rec * TR_H_ELEMS;
-        // blocked layouts: v = 32*jv + 8*q4 + e lies in value tile
-        // 2*jv + q4/2 at column 8*(q4%2) + e
-        const int64_t vnoff = (q4 >> 1) * TR_VN_TILE + x * 16 + 8 * (q4 & 1);
-        const uint16_t* vnrec = p.tr_vn + rec * TR_VN_ELEMS + vnoff;
-        const uint16_t* dvrec = p.tr_dvn + rec * TR_VN_ELEMS + vnoff;
-        const int xr = x < nvalid ? x : nvalid - 1;
-        const uint16_t* dorow = p.dout + ((sq.tok0 + c * BT + xr) * HV + hv) * DK + 8 * q4;
+        const uint16_t* vnrec = p.tr_vn + rec * TR_VN_ELEMS;
+        const uint16_t* dvrec = p.tr_dvn + rec * TR_VN_ELEMS;
+        const uint32_t hoff = (q4 >> 1) * TR_H_TILE + x * 16 + 8 * (q4 & 1);
+        const uint32_t vnoff = (q4 >> 1) * TR_VN_TILE + x * 16 + 8 * (q4 & 1);
+        const uint16_t* dobase = p.dout + (tok0 * HV + hv) * DK;
+        const uint32_t dooff = (uint32_t)(x < nvalid ? x : nvalid - 1) * (uint32_t)(HV * DK) + 8 * q4;
 #pragma unroll
         for (int jv = 0; jv < 4; ++jv) {
-            o.a_do[jv] = *reinterpret_cast<const u32x4*>(dorow + 32 * jv);
-            o.a_dv[jv] = *reinterpret_cast<const u32x4*>(dvrec + 2 * jv * TR_VN_TILE);
-            o.a_vn[jv] = *reinterpret_cast<const u32x4*>(vnrec + 2 * jv * TR_VN_TILE);
+            if (rows) {
+                o.a_do[jv] = *reinterpret_cast<const u32x4*>(dobase + 32 * jv + dooff);
+                o.a_dv[jv] = *reinterpret_cast<const u32x4*>(dvrec + 2 * jv * TR_VN_TILE + vnoff);
+                o.a_vn[jv] = *reinterpret_cast<const u32x4*>(vnrec + 2 * jv * TR_VN_TILE + vnoff);
+            }
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                const int kt = 2 * w + tt;
-                const int64_t off = (2 * jv + (q4 >> 1)) * TR_H_TILE + (16 * kt + x) * 16 +
-                                    8 * (q4 & 1);
-                o.bh[jv][tt] = *reinterpret_cast<const u32x4*>(hrec + off);
-                o.bd[jv][tt] = *reinterpret_cast<const u32x4*>(dhrec + off);
+            for (int tt = 0; tt < 2 && tiles; ++tt) {
+                const int base = 2 * jv * TR_H_TILE + (2 * w + tt) * 256;  // k-tile 2w + tt
+                o.bh[jv][tt] = *reinterpret_cast<const u32x4*>(hrec + base + hoff);
+                o.bd[jv][tt] = *reinterpret_cast<const u32x4*>(dhrec + base + hoff);
             }
         }
     };
@@ -268,12 +283,20 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
 
     // ---- q^, k^ (kernels.py:108-113), once per q/k head; the raw rows stay
     // packed and q^ / k^ are re-formed where needed --------------------------
-    const u32x4 qraw = *reinterpret_cast<const u32x4*>(p.q + (tokc * H + h) * DK + c0);
-    const u32x4 kraw = *reinterpret_cast<const u32x4*>(p.k + (tokc * H + h) * DK + c0);
+    u32x4 qraw, kraw;
+    auto load_qk = [&] {
+        const int64_t row = tok0 * H + h;
+        const uint32_t off = rowc() * (uint32_t)(H * DK) + c0;
+        qraw = *reinterpret_cast<const u32x4*>(p.q + row * DK + off);
+        kraw = *reinterpret_cast<const u32x4*>(p.k + row * DK + off);
+    };
+    load_qk();
     HvRaw hraw;
     HdhOps ops;
-    load_ops(h * rep, ops);
-    load_hv(h * rep, hraw);
+    if constexpr (!GROUP) {
+        load_ops(h, ops, true, true);
+        load_hv(h, hraw);
+    }
     float rq = 1.f, rk = 1.f;
     if (p.use_l2norm) {
         float qv[8], kv[8];
@@ -312,15 +335,35 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
     const int nrep = GROUP ? rep : 1;
     for (int gi = 0; gi < nrep; ++gi) {
         const int hv = h * rep + gi;
-        if (gi > 0) {
-            load_ops(hv, ops);
+        if constexpr (GROUP) {
+            // The thread's coordinates, the norms and the row count pass
+            // through opaque statements, so that what follows from them is
+            // formed in each iteration and not held across it.
+            asm volatile("" : "+v"(t), "+v"(rq), "+v"(rk));
+            if (!FULL) {
+                asm volatile("" : "+s"(nvalid));
+                mid = min(BT / 2, nvalid - 1);
+                last = nvalid - 1;
+            }
+            lane = t & 63;
+            x = lane & 15;
+            q4 = lane >> 4;
+            i = t >> 4;
+            cb = t & 15;
+            c0 = 8 * cb;
+            load_qk();  // (again, from the caches, rather than held)
+        }
+        // (in every iteration: loads before the loop for its first one only
+        // would keep their registers through the whole body)
+        if constexpr (GROUP) {
+            load_ops(hv, ops, false, true);
             load_hv(hv, hraw);
         }
         HvRow hr;
         decode_hv(hraw, hr);
         const SeqSpan sp = seq_span(p, seq * HV + hv);
         const int64_t rec = sp.rec0 + c;
-        const int64_t vrow = (tok * HV + hv) * DK;  // v/g/dO element offset of row i
+        const int64_t bi0 = tok0 * HV + hv;           // beta element of the chunk's first row
 
         // ---- phase 1: gates, cumsum, recentred operands; the matrix-op
         // operands of phase 2 are loaded meanwhile ---------------------------
@@ -375,15 +418,17 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
         __syncthreads();  // gm, gl
         {
             float E[8], eq[8], ek[8], kgl[8], qn[8], kn[8], o1[8], o2[8], o3[8], o4[8], o5[8];
+            float vr[8];
             gates(E, eq, ek, kgl);
             qk_hat(qn, kn);
+            row_v(hraw.v, vr);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 o1[j] = qn[j] * eq[j];
                 o2[j] = kn[j] * eq[j];
                 o3[j] = kn[j] * ek[j];
                 o4[j] = round_bf(round_bf(kn[j] * beta) * E[j]);
-                o5[j] = round_bf(hr.v[j] * beta);
+                o5[j] = round_bf(vr[j] * beta);
             }
             lds_put8(&sm.qp[i][c0], o1);
             lds_put8(&sm.kp[i][c0], o2);
@@ -394,6 +439,7 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
         __syncthreads();  // G is read; phase 2 overwrites dqg
 
         // ---- phase 2: products over V on the matrix cores ----------------
+        if constexpr (GROUP) load_ops(hv, ops, true, false);
         mask_ops(ops);
         // Wave w owns k-tiles 2w, 2w+1.  Lane (x, q4) feeds row x of dO /
         // dv_new / v_new and row 16*kt + x of h / dh', v columns
@@ -565,7 +611,8 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
             lds_get8(&sm.dvn[i][c0], dvb);
             lds_get8(&sm.dqg[i][c0], dqg);
             lds_get8(&sm.dkg[i][c0], dkg);
-            float dbeta = 0.f, kgkg[8];
+            float dbeta = 0.f, kgkg[8], vr[8];
+            row_v(hraw.v, vr);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const float qp = qn[j] * eq[j], kp = kn[j] * eq[j], km = kn[j] * ek[j];
@@ -574,7 +621,7 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
                 dQN[j] += dqg[j] * E[j] + dqp[j] * eq[j];
                 dKN[j] += dkb[j] * beta * E[j] + dkg[j] * kgl[j] + dkp[j] * eq[j] + dkm[j] * ek[j];
                 dbeta = fmaf(dkb[j], kn[j] * E[j], dbeta);
-                dbeta = fmaf(dvb[j], hr.v[j], dbeta);
+                dbeta = fmaf(dvb[j], vr[j], dbeta);
                 dv[j] = dvb[j] * beta;
                 const float d = LN2 * (dkb[j] * kb + dqg[j] * qg - dkg[j] * kg + dqp[j] * qp +
                                        dkp[j] * kp - dkm[j] * km);
@@ -583,12 +630,12 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
             }
             dbeta = row_sum16(dbeta) + dbl;
             if (valid) {
-                store8(p.dv + vrow + c0, dv);
+                store8(p.dv + bi0 * DK + (uint32_t)(i * HV * DK + c0), dv);
                 if (cb == 0) {
                     const float db = p.use_beta_sigmoid ? dbeta * beta * (1.f - beta) : dbeta;
-                    const int64_t bi = tok * HV + hv;
-                    if (p.beta_bf16) static_cast<uint16_t*>(p.dbeta)[bi] = f2bf(db);
-                    else static_cast<float*>(p.dbeta)[bi] = db;
+                    const uint32_t o = i * HV;
+                    if (p.beta_bf16) (static_cast<uint16_t*>(p.dbeta) + bi0)[o] = f2bf(db);
+                    else (static_cast<float*>(p.dbeta) + bi0)[o] = db;
                 }
             }
             // kp and km (dkp, dkm) are read only by their owning thread here
@@ -644,9 +691,9 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
             }
             if (valid) {
                 if (p.g_bf16) {
-                    store8(static_cast<uint16_t*>(p.dg) + vrow + c0, dg);
+                    store8(static_cast<uint16_t*>(p.dg) + bi0 * DK + (uint32_t)(i * HV * DK + c0), dg);
                 } else {
-                    float* dst = static_cast<float*>(p.dg) + vrow + c0;
+                    float* dst = static_cast<float*>(p.dg) + bi0 * DK + (uint32_t)(i * HV * DK + c0);
                     *reinterpret_cast<f32x4*>(dst) = f32x4{dg[0], dg[1], dg[2], dg[3]};
                     *reinterpret_cast<f32x4*>(dst + 4) = f32x4{dg[4], dg[5], dg[6], dg[7]};
                 }
@@ -680,6 +727,7 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
     }
 
     // ---- l2norm backward, dq / dk summed over the group -------------------
+    if constexpr (GROUP) load_qk();
     if (p.use_l2norm) {
         float qv[8], kv[8];
         unpack8(qraw, qv);
@@ -699,8 +747,9 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(GROUP ? 1 : 
         }
     }
     if (valid) {
-        store8(p.dq + (tok * H + h) * DK + c0, dQN);
-        store8(p.dk + (tok * H + h) * DK + c0, dKN);
+        const uint32_t off = i * H * DK + c0;
+        store8(p.dq + (tok0 * H + h) * DK + off, dQN);
+        store8(p.dk + (tok0 * H + h) * DK + off, dKN);
     }
 }
 
