@@ -1102,14 +1102,8 @@ __global__ __launch_bounds__(MODE == K2_FWD || MODE == K2_FWD_MS ? 192 : 256) vo
         }
         __builtin_amdgcn_endpgm();
     }
-    const int nbh = (p.cu_seqlens ? p.N : p.B) * p.HV;
-
-    // Work-group -> (head, value tile), XCD aware: consecutive work-group ids
-    // go to different XCDs round-robin, so the 8 tiles of one head get ids
-    // of one residue class mod 8 and share that XCD's L2 for the records.
-    const int wg = blockIdx.x;
-    const int lin = (wg & 7) * nbh + (wg >> 3);
-    const int bh = lin >> 3;  // (batch row or sequence) * HV + value head
+    int bh, vt;  // (batch row or sequence) * HV + value head, its value tile
+    if (!k2_pair<8>(p, blockIdx.x, bh, vt)) __builtin_amdgcn_endpgm();  // padding: before any barrier
     const int hv = bh - (bh / p.HV) * p.HV;
     const SeqSpan sp = seq_span(p, bh);
 
@@ -1119,7 +1113,7 @@ __global__ __launch_bounds__(MODE == K2_FWD || MODE == K2_FWD_MS ? 192 : 256) vo
     cx.T = sp.len;
     cx.lane = lane;
     cx.q4 = lane >> 4;
-    cx.vt = lin & 7;
+    cx.vt = vt;
     cx.rev = MODE == K2_BWD;
     cx.ut = 0;
 
@@ -1174,14 +1168,8 @@ __global__ __launch_bounds__(64 * (TPW + 2)) void k2s_kernel(Params p) {
     constexpr int NSL = 8 / TPW;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nbh = (p.cu_seqlens ? p.N : p.B) * p.HV;
-    const int total = nbh * NSL;
-    const int padded = (total + 8 * NSL - 1) / (8 * NSL) * (8 * NSL);
-    const int wg = blockIdx.x;
-    const int lin = (wg & 7) * (padded >> 3) + (wg >> 3);
-    if (lin >= total) return;  // padding: the whole work-group leaves before any barrier
-    const int bh = lin / NSL;
-    const int slice = lin - bh * NSL;
+    int bh, slice;
+    if (!k2_pair<NSL>(p, blockIdx.x, bh, slice)) return;  // padding: the whole work-group leaves before any barrier
     const int hv = bh - (bh / p.HV) * p.HV;
     const SeqSpan sp = seq_span(p, bh);
 
@@ -1239,6 +1227,12 @@ static int cu_count() {
     return cached[dev];
 }
 
+// Work-groups of a stage 2 with NSL slices a head (k2_pair).
+static unsigned k2_grid(const Params& p, int nsl) {
+    const int64_t nbh = (int64_t)(p.cu_seqlens ? p.N : p.B) * p.HV;
+    return (unsigned)(nsl == 8 && !p.cu_seqlens ? nbh * 8 : (nbh + 7) / 8 * 8 * nsl);
+}
+
 hipError_t launch_k2(const Params& p, hipStream_t stream) {
     const int nseq = p.cu_seqlens ? p.N : p.B;
     const int64_t tiles = (int64_t)p.HV * 8;
@@ -1250,9 +1244,7 @@ hipError_t launch_k2(const Params& p, hipStream_t stream) {
     // or a caller's k2_wave_tiles: kda_k2w.hip.
     if (const int tpw = k2_wide_tiles(p, ncu)) {
         if (tpw == 2 && p.k2_wave_tiles == 0) {
-            const int64_t nbh = (int64_t)(p.cu_seqlens ? p.N : p.B) * p.HV;
-            const int64_t padded = (nbh * 4 + 31) / 32 * 32;  // 4 slices a head, 8 XCDs
-            hipLaunchKernelGGL(k2s_kernel<2>, dim3((unsigned)padded), dim3(64 * 4), 0, stream, p);
+            hipLaunchKernelGGL(k2s_kernel<2>, dim3(k2_grid(p, 4)), dim3(64 * 4), 0, stream, p);
             return hipGetLastError();
         }
         return launch_k2_wide(p, tpw, stream);
@@ -1266,8 +1258,7 @@ hipError_t launch_k2(const Params& p, hipStream_t stream) {
                            stream, q);
         return hipGetLastError();
     }
-    const int64_t grid = nseq * tiles;
-    hipLaunchKernelGGL(k2_kernel<K2_FWD>, dim3((unsigned)grid), dim3(192), 0, stream, p);
+    hipLaunchKernelGGL(k2_kernel<K2_FWD>, dim3(k2_grid(p, 8)), dim3(192), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -1386,20 +1377,17 @@ hipError_t launch_fwd_save(const Params& p, hipStream_t stream) {
 }
 
 hipError_t launch_k2_train(const Params& p, hipStream_t stream) {
-    const int64_t grid = (int64_t)(p.cu_seqlens ? p.N : p.B) * p.HV * 8;
-    hipLaunchKernelGGL(k2_kernel<K2_TRAIN>, dim3((unsigned)grid), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(k2_kernel<K2_TRAIN>, dim3(k2_grid(p, 8)), dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 
 hipError_t launch_k2_train_o(const Params& p, hipStream_t stream) {
-    const int64_t grid = (int64_t)(p.cu_seqlens ? p.N : p.B) * p.HV * 8;
-    hipLaunchKernelGGL(k2_kernel<K2_TRAIN_O>, dim3((unsigned)grid), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(k2_kernel<K2_TRAIN_O>, dim3(k2_grid(p, 8)), dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 
 hipError_t launch_k2_bwd(const Params& p, hipStream_t stream) {
-    const int64_t grid = (int64_t)(p.cu_seqlens ? p.N : p.B) * p.HV * 8;
-    hipLaunchKernelGGL(k2_kernel<K2_BWD>, dim3((unsigned)grid), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(k2_kernel<K2_BWD>, dim3(k2_grid(p, 8)), dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -11,6 +11,60 @@ namespace {
 
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
 
+// The sequence of rank s when the N packed sequences are ordered longest
+// first (up to 64 sequences; beyond that, or past the last, s itself).
+__device__ __forceinline__ int longest_first(const Params& p, int s) {
+    if (p.N > 64) return s;
+    const int lane = threadIdx.x & 63;
+    const int len = lane < p.N ? cu_at(p, lane + 1) - cu_at(p, lane) : -1;
+    // rank of this lane's sequence: the sequences longer, or as long with a
+    // lower index
+    int rank = 0;
+    for (int m = 0; m < p.N; ++m) {
+        const int lm = __builtin_amdgcn_readlane(len, m);
+        rank += (lm > len || (lm == len && m < lane)) ? 1 : 0;
+    }
+    const uint64_t hit = __ballot(lane < p.N && rank == s);
+    if (hit == 0) return s;  // (the ranks are a permutation: past the last only)
+    return __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(hit));
+}
+
+// Stage 2's work-group -> (sequence or batch row, value head) bh and slice of
+// the head's value tiles, NSL slices a head, XCD aware: work-group ids go to
+// the XCDs round-robin, so the slices of a head, on ids of one residue class
+// mod 8, share that XCD's L2 for the records.  Batch rows: XCD x takes the
+// x-th eighth of the work-groups.  Packed sequences, whose chains differ in
+// length: the heads are dealt to the XCDs in turn and, where the work-groups
+// outnumber the CUs, longest sequences first, so that each XCD has its share
+// of every sequence and starts its longest chains at once.  (An eighth of the
+// heads each put whole sequences on one XCD: 6 sequences of 33 to 1311 tokens,
+// HV = 16, the training forward's stage 2 109 us against 68, the reverse chain
+// 129 against 90.  Where all work-groups start at once their order does not
+// matter, and finding it costs a load and ~1 us.)  False past the last head
+// (grid: k2_grid).
+constexpr int CU_COUNT = 256;
+template <int NSL>
+__device__ __forceinline__ bool k2_pair(const Params& p, int wg, int& bh, int& slice) {
+    const int nbh = (p.cu_seqlens ? p.N : p.B) * p.HV;
+    const int xcd = wg & 7, j = wg >> 3;
+    if (p.cu_seqlens) {
+        slice = j % NSL;
+        const int idx = (j / NSL) * 8 + xcd;
+        if (idx >= nbh) return false;
+        bh = idx;
+        if (nbh * NSL > CU_COUNT) {
+            const int s = idx / p.HV;
+            bh = longest_first(p, s) * p.HV + (idx - s * p.HV);
+        }
+        return true;
+    }
+    const int total = nbh * NSL;
+    const int lin = xcd * (NSL == 8 ? nbh : (total + 8 * NSL - 1) / (8 * NSL) * NSL) + j;
+    bh = lin / NSL;
+    slice = lin - bh * NSL;
+    return lin < total;
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N));

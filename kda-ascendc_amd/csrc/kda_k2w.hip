@@ -124,14 +124,8 @@ __global__ __launch_bounds__((WideGeom<TPW, TW>::THREADS)) void k2w_kernel(Param
     constexpr int NSL = 8 / TPW;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nbh = (p.cu_seqlens ? p.N : p.B) * p.HV;
-    const int total = nbh * NSL;
-    const int padded = (total + 8 * NSL - 1) / (8 * NSL) * (8 * NSL);
-    const int wg = blockIdx.x;
-    const int lin = (wg & 7) * (padded >> 3) + (wg >> 3);
-    if (lin >= total) return;  // padding: the whole work-group leaves before any barrier
-    const int bh = lin / NSL;
-    const int slice = lin - bh * NSL;
+    int bh, slice;
+    if (!k2_pair<NSL>(p, blockIdx.x, bh, slice)) return;  // padding: the whole work-group leaves before any barrier
     const int hv = bh - (bh / p.HV) * p.HV;
     const SeqSpan sp = seq_span(p, bh);
     const int64_t sbase = (int64_t)bh * DK * DK;
