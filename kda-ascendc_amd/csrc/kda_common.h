@@ -346,6 +346,11 @@ __device__ __forceinline__ float row_sum16(float x) {
     return x;
 }
 
+// The wave's own LDS writes are complete before its next LDS read: the
+// scratch of k1_chunk belongs to one wave, so no work-group barrier is
+// needed between its phases.
+__device__ __forceinline__ void wave_lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // The value of lane ^ 16 (within each 32 lanes), by ds_swizzle in bit mode:
 // and_mask 0x1f, or_mask 0, xor_mask 0x10.
 __device__ __forceinline__ float xor16(float x) {

@@ -94,11 +94,6 @@ struct K1Scratch {
     uint8_t* kg;  // TILE_BYTES
 };
 
-// The wave's own LDS writes are complete before its next LDS read: the
-// scratch of k1_chunk belongs to one wave, so no work-group barrier is
-// needed between its phases.
-__device__ __forceinline__ void wave_lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
 // Record modes.  K1_FWD: the forward record.  K1_BOTH (the backward's
 // recompute): the forward record without qg (no o is formed), the gram
 // block in qg's bytes, and the backward record with dO.  K1_SAVE (a

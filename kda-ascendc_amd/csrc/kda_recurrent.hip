@@ -16,7 +16,12 @@
 // decode step (README.md:503-505).  No rounding happens between tokens, so
 // with o in fp32 the kernel is also an on-GPU gold for the chunked path.
 //
-// One work-group of 256 threads per (sequence or batch row, value head).
+// Two kernels, which give the same bits.  recurrent_kernel: the decode step and
+// fixed-length calls of two or three tokens whose states fill the chip, where the
+// states' bytes bound the call; recurrent_rows_kernel, below: everything else, bound
+// by the latency of the tokens.
+//
+// recurrent_kernel: one work-group of 256 threads per (batch row, value head).
 // Thread t = 32 * hw + j holds the 64 state elements at memory offsets
 // 1024 * i + 4 * t + c (i = 0..15, c = 0..3) of the head's 128 x 128 state,
 // so every state load and store is a 16-byte access and each wave
@@ -29,10 +34,10 @@
 //     over i in registers, then over the eight half-waves: lane pairs of a
 //     wave by a shuffle, the four waves through LDS.
 // The state lives in registers for the whole sequence (64 floats per
-// thread, 165 VGPRs in all), so three work-groups share a CU and the decode
-// step streams the states at close to the memory system's rate.
+// thread; 106 to 161 VGPRs in all), so three or four work-groups share a CU and the
+// decode step streams the states at close to the memory system's rate.
 // Grouped value heads (GVA): value head hv reads q/k head hv / (HV / H)
-// (kernels.py:88).  Varlen: one work-group per (sequence, value head), over
+// (kernels.py:88).  Varlen: the work-groups of a (sequence, value head) go over
 // the sequence's tokens, with states [N, HV, ...].
 #include "kda_common.h"
 
@@ -148,7 +153,7 @@ __device__ __forceinline__ void store_o(const Params& p, int64_t idx, float x) {
 template <bool VFIRST, bool ONE>
 __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(ONE ? 4 : 1))) void recurrent_kernel(Params p) {
     const int HV = p.HV, H = p.H;
-    const int bhv = blockIdx.x;  // (batch row or sequence) * HV + hv
+    const int bhv = blockIdx.x;  // batch row * HV + hv
     const int hv = bhv - (bhv / HV) * HV;
     const int h = hv / (HV / H);
     const SeqSpan sp = seq_span(p, bhv);
@@ -328,14 +333,287 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(ONE ? 4 : 1)
     }
 }
 
+// Several tokens.  The rows of S are independent of each other, so SPLIT
+// work-groups share a (sequence, value head) and each of a work-group's SW state
+// waves takes 16 rows v: lane (x, g), x = lane % 16, g = lane / 16, holds row
+// v = x's 32 elements of column group g, both products of a token are 32 FMAs in
+// registers and a sum over the four groups, and no state wave waits for another.
+// SF further waves, the formers, take the expf, the divisions and the loads: they
+// form the decays, k^, q^, beta and v of the next SF tokens, a token each, in the
+// other one of two LDS buffers; one barrier every SF tokens.
+//
+// Bound by the latency of a token's chain (LDS reads, 32 products, the exchange,
+// the update, 32 products), 0.75 us a token where recurrent_kernel's reductions
+// across lanes (V-first) or waves (K-first) take 2.1 (K-first) to 3.1 (V-first).
+// Four sequences of 24 tokens at 16 heads: 57 -> 26 us K-first, 81 -> 25 V-first;
+// with the chip full, 2048 (sequence, head) pairs of 24 tokens: 232 -> 196 and
+// 316 -> 178.  Two waves a side instead of four: V-first 244 (the formers are
+// late); one former per work-group: 31 and 38 at the small size.
+// 107 VGPRs, 47 KB of LDS: two work-groups a CU.
+//
+// The column groups and the order of the sums are recurrent_kernel's, so that
+// the two, and T decode steps and one call of T tokens, give the same bits:
+//   V-first: group g holds k = 32*g .. +31, as eight partial sums of four, added
+//     as half_sum adds lanes 8*g .. 8*g + 7, then the groups as it adds the rest;
+//   K-first: group g holds k = 8*i + 2*g + {0, 1}, one chain over i each, their
+//     sum, then ((g0 + g1) + g2) + g3.
+constexpr int SW = 4, SF = 4;
+static_assert(16 * SW == 64, "a former's lanes load the work-group's v");
+constexpr int SPLIT = DK / (16 * SW);
+constexpr int VEC_GROUP = 36;  // floats between column groups in LDS (no bank conflicts)
+
+// The sum over the four column groups, in every lane.
+template <bool VFIRST>
+__device__ __forceinline__ float group_sum(float r) {
+    const auto swap16 = [](float x) {
+        const uint32_t b = __builtin_bit_cast(uint32_t, x);
+        return __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    };
+    const auto swap32 = [](uint32_t b) { return __builtin_amdgcn_permlane32_swap(b, b, false, false); };
+    const auto f = [](uint32_t b) { return __builtin_bit_cast(float, b); };
+    const auto p = swap16(r);  // the groups 0, 0, 2, 2 and 1, 1, 3, 3 of the lane's row
+    if constexpr (VFIRST) {
+        const auto h = swap32(__builtin_bit_cast(uint32_t, f(p[0]) + f(p[1])));
+        return f(h[0]) + f(h[1]);
+    } else {
+        const auto e = swap32(p[0]), o = swap32(p[1]);
+        return f(e[0]) + f(o[0]) + f(e[1]) + f(o[1]);
+    }
+}
+
+// This lane's part of the product of its 32 elements with a vector.
+template <bool VFIRST>
+__device__ __forceinline__ float group_part(const f32x4 (&S)[8], const f32x4 (&y)[8]) {
+    if constexpr (VFIRST) {
+        float q[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            q[m] = 0.f;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) q[m] = fmaf(S[m][c], y[m][c], q[m]);
+        }
+        return ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
+    } else {
+        float e = 0.f, o = 0.f;  // k even and odd
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            e = fmaf(S[m][0], y[m][0], e);
+            o = fmaf(S[m][1], y[m][1], o);
+            e = fmaf(S[m][2], y[m][2], e);
+            o = fmaf(S[m][3], y[m][3], o);
+        }
+        return e + o;
+    }
+}
+
+// A token's raw inputs for a lane of a former.  V-first: q and k at columns
+// 4j .. 4j+3, j = lane % 32 (the norms are summed in this order), the rest for
+// columns 4j + 2*(lane / 32) + {0, 1}; K-first: columns 2*lane + {0, 1}.  gp: the
+// previous token's g, of the cumsum form.
+struct FormRaw {
+    u32x2 q, k;
+    f32x2 g, gp;
+    float beta;
+    uint16_t v;  // row v0 + lane
+};
+
+template <bool VFIRST>
+__device__ __forceinline__ f32x2 load_g2(const Params& p, int64_t at) {
+    if (p.g_bf16) {
+        const uint32_t w = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(p.g) + at);
+        return f32x2{lo16(w), hi16(w)};
+    }
+    return *reinterpret_cast<const f32x2*>(static_cast<const float*>(p.g) + at);
+}
+
+template <bool VFIRST>
+__device__ __forceinline__ void load_form(const Params& p, const SeqSpan& sp, int tt, int h, int hv, int lane,
+                                          int col, int v0, FormRaw& r) {
+    const int64_t rq = (sp.tok0 + tt) * p.H + h;
+    const int64_t rv = (sp.tok0 + tt) * p.HV + hv;
+    if constexpr (VFIRST) {
+        r.q = *reinterpret_cast<const u32x2*>(p.q + rq * DK + 4 * (lane & 31));
+        r.k = *reinterpret_cast<const u32x2*>(p.k + rq * DK + 4 * (lane & 31));
+    } else {
+        r.q.x = *reinterpret_cast<const uint32_t*>(p.q + rq * DK + col);
+        r.k.x = *reinterpret_cast<const uint32_t*>(p.k + rq * DK + col);
+    }
+    r.g = load_g2<VFIRST>(p, rv * DK + col);
+    r.gp = f32x2{0.f, 0.f};
+    if (!p.use_gate && !p.g_log && tt % BT != 0) r.gp = load_g2<VFIRST>(p, (rv - p.HV) * DK + col);
+    r.beta = load_scalar(p.beta, p.beta_bf16, rv);
+    r.v = p.v[rv * DK + v0 + lane];
+}
+
+// A vector's two columns of the lane, divided by its norm.
+template <bool VFIRST>
+__device__ __forceinline__ f32x2 unit2(const Params& p, u32x2 w, int lane) {
+    f32x2 y;
+    if constexpr (VFIRST) {
+        const uint32_t mine = lane < 32 ? w.x : w.y;
+        y = f32x2{lo16(mine), hi16(mine)};
+    } else {
+        y = f32x2{lo16(w.x), hi16(w.x)};
+    }
+    if (!p.use_l2norm) return y;
+    float ss;
+    if constexpr (VFIRST) {
+        const float c[4] = {lo16(w.x), hi16(w.x), lo16(w.y), hi16(w.y)};
+        ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ss = fmaf(c[i], c[i], ss);
+        ss = half_sum(ss);
+    } else {
+        ss = half_sum(fmaf(y.x, y.x, y.y * y.y));
+        ss += __shfl_xor(ss, 32, 64);
+    }
+    const float n = sqrtf(ss + L2_EPS);
+    return f32x2{y.x / n, y.y / n};
+}
+
+template <bool VFIRST>
+__global__ __launch_bounds__(64 * (SW + SF)) void recurrent_rows_kernel(Params p) {
+    const int HV = p.HV;
+    const int bhv = blockIdx.x / SPLIT;  // (batch row or sequence) * HV + hv
+    const int hv = bhv - (bhv / HV) * HV;
+    const SeqSpan sp = seq_span(p, bhv);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int len = sp.len;
+
+    // The vectors of two times SF tokens: decay, k^, q^, each as four groups of
+    // 32, and beta.
+    __shared__ __attribute__((aligned(16))) float s_vec[2][SF][3][4 * VEC_GROUP];
+    __shared__ float s_beta[2][SF], s_v[2][SF][16 * SW];
+    // V-first: a wave's 16 rows on their way between memory, which is read and
+    // written in whole KiB, and the lanes; unit u (16 bytes) of row r at u ^ r.
+    __shared__ __attribute__((aligned(16))) float s_rows[VFIRST ? SW : 1][VFIRST ? 16 * DK : 4];
+
+    const int v0 = (blockIdx.x % SPLIT) * 16 * SW;  // the work-group's rows
+    if (wave >= SW) {
+        const int f = wave - SW;
+        const int h = hv / (HV / p.H);
+        const float ea = p.use_gate ? expf(p.A_log[hv]) : 0.0f;
+        const int j = lane & 31;
+        const int col = VFIRST ? 4 * j + 2 * (lane >> 5) : 2 * lane;
+        const int at = VFIRST ? (j >> 3) * VEC_GROUP + (col & 31) : (lane & 3) * VEC_GROUP + 2 * (lane >> 2);
+        f32x2 dtb = {0.f, 0.f};
+        if (p.use_gate && p.dt_bias) dtb = f32x2{p.dt_bias[hv * DK + col], p.dt_bias[hv * DK + col + 1]};
+        FormRaw cur, nxt;
+        if (len > 0) load_form<VFIRST>(p, sp, min(f, len - 1), h, hv, lane, col, v0, cur);
+        for (int t0 = 0; t0 < len; t0 += SF) {
+            // (past the end the last token again: it is formed and not read)
+            load_form<VFIRST>(p, sp, min(t0 + SF + f, len - 1), h, hv, lane, col, v0, nxt);
+            const int buf = (t0 / SF) & 1;
+            float (*vec)[4 * VEC_GROUP] = s_vec[buf][f];
+            f32x2 a;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                float gp = cur.gp[c];
+                a[c] = decay_of(p, cur.g[c], ea, dtb[c], gp, false);
+            }
+            *reinterpret_cast<f32x2*>(&vec[0][at]) = a;
+            *reinterpret_cast<f32x2*>(&vec[1][at]) = unit2<VFIRST>(p, cur.k, lane);
+            *reinterpret_cast<f32x2*>(&vec[2][at]) = unit2<VFIRST>(p, cur.q, lane);
+            if (lane == 0) s_beta[buf][f] = p.use_beta_sigmoid ? sigmoid_precise(cur.beta) : cur.beta;
+            s_v[buf][f][lane] = bf2f(cur.v);
+            // tokens t0 .. t0 + SF - 1 are formed, and those before them, whose
+            // buffer the next ones take, have been read
+            __syncthreads();
+            cur = nxt;
+        }
+        return;
+    }
+
+    const int x = lane & 15, g = lane >> 4;
+    const int v = v0 + 16 * wave + x;
+    const int64_t sbase = (int64_t)bhv * DK * DK;
+    // V-first: the wave's rows, lane by lane in order of memory, and the lane's
+    // element 4*m, k = 32*g + 4*m; K-first element 2*i + e: k = 8*i + 2*g + e
+    float* rows = s_rows[VFIRST ? wave : 0];
+    const int half = lane >> 5;
+    int unit = lane & 31, xs = x;
+    auto linear = [&](int m) { return rows + (2 * m + half) * DK + 4 * (unit ^ (2 * m + half)); };
+    auto mine = [&](int m) { return rows + xs * DK + 4 * ((8 * g + m) ^ xs); };
+    const int64_t slab = sbase + (int64_t)(v - x) * DK + 4 * lane;
+    auto element = [&](int n) { return sbase + (8 * (n >> 1) + 2 * g + (n & 1)) * DK + v; };
+    f32x4 S[8] = {};
+    if (p.h0) {
+        if constexpr (VFIRST) {
+#pragma unroll
+            for (int m = 0; m < 8; ++m) S[m] = *reinterpret_cast<const f32x4*>(p.h0 + slab + 256 * m);
+#pragma unroll
+            for (int m = 0; m < 8; ++m) *reinterpret_cast<f32x4*>(linear(m)) = S[m];
+            wave_lds_fence();
+#pragma unroll
+            for (int m = 0; m < 8; ++m) S[m] = *reinterpret_cast<const f32x4*>(mine(m));
+        } else {
+#pragma unroll
+            for (int n = 0; n < 32; ++n) S[n >> 2][n & 3] = p.h0[element(n)];
+        }
+    }
+    const int64_t row0 = sp.tok0 * HV + hv;
+    for (int t0 = 0; t0 < len; t0 += SF) {
+        __syncthreads();  // tokens t0 .. t0 + SF - 1 are formed
+        const int buf = (t0 / SF) & 1, n = min(SF, len - t0);
+#pragma unroll 1
+        for (int f = 0; f < n; ++f) {
+            const float (*vec)[4 * VEC_GROUP] = s_vec[buf][f];
+            f32x4 kv[8], qv[8];
+#pragma unroll
+            for (int m = 0; m < 8; ++m) {
+                const f32x4 a = *reinterpret_cast<const f32x4*>(&vec[0][g * VEC_GROUP + 4 * m]);
+                kv[m] = *reinterpret_cast<const f32x4*>(&vec[1][g * VEC_GROUP + 4 * m]);
+                S[m] = S[m] * a;
+            }
+            const float pred = group_sum<VFIRST>(group_part<VFIRST>(S, kv));
+#pragma unroll
+            for (int m = 0; m < 8; ++m) qv[m] = *reinterpret_cast<const f32x4*>(&vec[2][g * VEC_GROUP + 4 * m]);
+            const float vnew = s_beta[buf][f] * (s_v[buf][f][16 * wave + x] - pred);
+#pragma unroll
+            for (int m = 0; m < 8; ++m) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) S[m][c] = fmaf(vnew, kv[m][c], S[m][c]);
+            }
+            const float o = group_sum<VFIRST>(group_part<VFIRST>(S, qv));
+            if (g == 0) store_o(p, (row0 + (int64_t)(t0 + f) * HV) * DK + v, p.scale * o);
+        }
+    }
+    if (p.ht) {
+        asm("" : "+v"(unit), "+v"(xs));  // (their addresses are formed again, not kept through the loop)
+        if constexpr (VFIRST) {
+#pragma unroll
+            for (int m = 0; m < 8; ++m) *reinterpret_cast<f32x4*>(mine(m)) = S[m];
+            wave_lds_fence();
+#pragma unroll
+            for (int m = 0; m < 8; ++m)
+                *reinterpret_cast<f32x4*>(p.ht + slab + 256 * m) = *reinterpret_cast<const f32x4*>(linear(m));
+        } else {
+#pragma unroll
+            for (int n = 0; n < 32; ++n) p.ht[element(n)] = S[n >> 2][n & 3];
+        }
+    }
+}
+
 }  // namespace
 
 hipError_t launch_recurrent(const Params& p, hipStream_t stream) {
-    const int64_t grid = (int64_t)(p.cu_seqlens ? p.N : p.B) * p.HV;
+    const int64_t pairs = (int64_t)(p.cu_seqlens ? p.N : p.B) * p.HV;
+    // Two or three tokens with the chip full spend their time on the states, of
+    // which recurrent_kernel has three work-groups' 64 KB a CU in flight where
+    // recurrent_rows_kernel has two of 32: V-first, 4096 pairs, 123 us against 139 at two
+    // tokens; 2048 pairs, 103 against 84 at six.  K-first the two are equal at
+    // two tokens (125 us), and up to 512 pairs (one round) V-first ones are.
+    const bool few = !p.cu_seqlens && p.T <= 3 && p.h0_v_first && pairs > 512;
     const bool one = !p.cu_seqlens && p.T == 1;
+    if (!one && !few) {
+        auto rows = p.h0_v_first ? recurrent_rows_kernel<true> : recurrent_rows_kernel<false>;
+        hipLaunchKernelGGL(rows, dim3((unsigned)(pairs * SPLIT)), dim3(64 * (SW + SF)), 0, stream, p);
+        return hipGetLastError();
+    }
     auto kern = p.h0_v_first ? (one ? recurrent_kernel<true, true> : recurrent_kernel<true, false>)
-                             : (one ? recurrent_kernel<false, true> : recurrent_kernel<false, false>);
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(RT), 0, stream, p);
+                             : recurrent_kernel<false, true>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)pairs), dim3(RT), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -113,6 +113,7 @@ def kernel_role(name: str) -> str | None:
         return _K2_MODES.get(m.group(1), "k2_mode" + m.group(1))
     for key, role in (("fused_kernel", "fused"), ("k1_dout_kernel", "k1_dout"),
                       ("k2w_kernel", "k2"), ("k2s_kernel", "k2"), ("recurrent_kernel", "recurrent"),
+                      ("recurrent_rows_kernel", "recurrent"),
                       ("bwd_chunk_kernel", "bwd_chunk"), ("gate_segment_kernel", "gate_segment"),
                       ("gate_reduce_kernel", "gate_reduce"),
                       ("copyBuffer", "copy")):

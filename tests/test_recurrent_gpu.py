@@ -124,6 +124,38 @@ def test_decode_steps_equal_one_call(vfirst, gpu_device):
     assert torch.equal(state, ht_all)
 
 
+@pytest.mark.parametrize("B,T,HV,vfirst,packed", [
+    (16, 3, 32, True, False),   # 512 pairs: the row-split kernel
+    (19, 2, 27, True, False),   # 513 pairs, two and three tokens: the one-work-group kernel
+    (19, 3, 27, True, False),
+    (19, 4, 27, True, False),
+    (19, 3, 27, False, False),
+    (2, 5, 2, True, False),     # lengths around the four tokens formed at a time
+    (1, 8, 3, False, False),
+    (3, 1, 2, True, True),
+    (3, 4, 2, False, True),
+    (2, 17, 2, True, True),
+])
+def test_both_kernels_give_the_same_bits(B, T, HV, vfirst, packed, gpu_device):
+    """A call of T tokens (or of B packed sequences of T), whichever kernel
+    serves it, equals T decode steps bit for bit."""
+    dev = gpu_device
+    c = _inputs(B, T, HV, HV, seed=5 + T, gate_dtype=torch.bfloat16)
+    kw = dict(scale=0.1, use_qk_l2norm_in_kernel=True, use_gate_in_kernel=True,
+              use_beta_sigmoid_in_kernel=True, lower_bound=-5.0, A_log=c["A_log"].to(dev),
+              dt_bias=c["dt_bias"].to(dev), state_v_first=vfirst)
+    x = {n: c[n].to(dev) for n in ("q", "k", "v", "g", "beta")}
+    h0 = c["h0"].to(dev)
+    cu = torch.arange(0, (B + 1) * T, T, dtype=torch.int32, device=dev) if packed else None
+    ins = [t.flatten(0, 1)[None] if packed else t for t in x.values()]
+    o, ht = kda_recurrent_fwd(*ins, initial_state=h0, output_final_state=True, cu_seqlens=cu, **kw)
+    state = h0.clone()
+    steps = [kda_decode_step(*(t[:, i:i + 1].contiguous() for t in x.values()), state, **kw)
+             for i in range(T)]
+    assert torch.equal(o.reshape(B, T, HV, 128), torch.cat(steps, dim=1))
+    assert torch.equal(ht, state)
+
+
 def test_chunked_path_vs_gpu_gold_headline(gpu_device):
     """BASELINE configs[2] (B=1 T=8192 H=32, bf16 storage) against the GPU
     recurrence in fp32, pinned itself against the CPU gold on two heads."""
