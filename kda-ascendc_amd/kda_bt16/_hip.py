@@ -248,6 +248,6 @@ def call_saved(name: str, args, saved: int, nbytes: int, stream: int) -> None:
 
 
 def call(name: str, args, stream: int) -> None:
-    rc = getattr(lib(), name)(ctypes.byref(args), ctypes.c_void_p(stream))
+    rc = getattr(_lib or lib(), name)(ctypes.byref(args), stream)
     if rc != 0:
         raise KdaHipError(name, rc, lib().kda_bt16_strerror(rc).decode())

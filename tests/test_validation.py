@@ -262,3 +262,52 @@ def test_forward_choice_reaches_the_abi_arguments():
         assert seen[0].k2_tiles == 0
     a = args()
     assert not a.flags & (_hip.FUSED_KERNEL | _hip.TWO_STAGE) and a.k2_tiles == 0
+
+
+def _one_wrong(x, i):
+    """The call with its i-th form changed: ordinary forms first, then wrong ones."""
+    f32, bf16 = torch.float32, torch.bfloat16
+    forms = [
+        {}, {"g": x["g"].to(bf16)}, {"beta": x["beta"].to(bf16)}, {"initial_state": None},
+        {"A_log": None}, {"dt_bias": None}, {"use_gate": False, "A_log": None}, {"lower_bound": None},
+        {"lower_bound": 0.0}, {"lower_bound": -11.0}, {"lower_bound": float("nan")}, {"safe_gate": False},
+        {"use_gate": False, "g": x["g"].to(torch.float16)}, {"g": x["g"].to(torch.float16)},
+    ]
+    for n in ("q", "k", "v", "g", "beta", "initial_state", "A_log", "dt_bias"):
+        t = x[n]
+        forms += [{n: t.double()}, {n: t.to(torch.int32)}, {n: t[None]}, {n: t[:0]}, {n: t[..., :-1].contiguous()},
+                  {n: torch.cat([t, t], 0)}, {n: torch.cat([t, t], -1)[..., ::2]}, {n: t.flatten()}]
+        if t.ndim > 1:
+            forms += [{n: t.transpose(0, 1).contiguous()}, {n: t.transpose(-1, -2)}, {n: t[:, :0]}]
+    for n, d in (("q", bf16), ("k", bf16), ("v", bf16), ("A_log", f32)):
+        forms += [{n: x[n].to(f32 if d is bf16 else bf16)}]
+    forms += [{"q": x["q"][:, :, :0], "k": x["k"][:, :, :0]}, {"v": x["v"][:, :, :0]},
+              {n: x[n][:, :0] for n in ("q", "k", "v", "g", "beta")},
+              {n: x[n][..., :64].contiguous() for n in ("q", "k", "g")}]
+    return {**x, **forms[i]} if i < len(forms) else None
+
+
+@pytest.mark.parametrize("B,T,H,HV", [(1, 1, 1, 1), (2, 3, 2, 4), (1, 5, 2, 3)])
+def test_quick_checks_accept_only_what_the_full_checks_do(B, T, H, HV):
+    """What ``_plainly_valid`` accepts, the checks in the order of their
+    messages accept; and it does accept the ordinary call."""
+    from kda_bt16.kernels import _plainly_valid, _validate_kda_inputs
+
+    x = dict(q=torch.zeros(B, T, H, 128, dtype=torch.bfloat16), k=torch.zeros(B, T, H, 128, dtype=torch.bfloat16),
+             v=torch.zeros(B, T, HV, 128, dtype=torch.bfloat16), g=torch.zeros(B, T, HV, 128),
+             beta=torch.zeros(B, T, HV), initial_state=torch.zeros(B, HV, 128, 128), use_gate=True, safe_gate=True,
+             lower_bound=-5.0, A_log=torch.zeros(HV), dt_bias=torch.zeros(HV * 128))
+    i = 0
+    while (c := _one_wrong(x, i)) is not None:
+        for v_first in (True, False):
+            plain = _plainly_valid(*c.values())
+            try:
+                full = _validate_kda_inputs(*c.values(), v_first)
+            except (TypeError, ValueError) as e:
+                full = e
+            if plain:
+                assert full == (B, T, H, 128, HV, 128), (i, full)
+            if i < 4:
+                assert plain == (HV % H == 0), i
+        i += 1
+    assert i > 90
