@@ -194,8 +194,9 @@ struct Ctx {
     uint32_t u_lds;             // copy: REC_SHARED + 512 * (vt % 2), its place in a ring slot
     uint16_t* obase;            // output: o[first token, hv, 16*vt + 4*((lane%16)/4)]
     int64_t orow_stride;        // output: elements between consecutive tokens of o
-    uint16_t* trh;              // training: h of the first record, this tile, column 4*((lane%16)/4)
+    uint16_t* trh;              // training: h of the first record, the lane's place in this tile
     uint16_t* trvn;             // training: v_new of the first record, likewise
+    int tr_src, tr_vsrc;        // training: what the lane points the transposing reads of hc and v_new at
     int rev;                    // backward: step c handles chunk NT - 1 - c
     float scale;
     int NT, T, lane, q4, vt;    // NT chunks over T tokens (this sequence's)
@@ -373,40 +374,42 @@ __device__ __forceinline__ void state_step(const Ctx& cx, f32x4 (&St)[8], StateO
 #undef KDA_FENCE
 }
 
+// ds_read_b64_tr_b16 (the transpose: see output_step).
+__device__ __forceinline__ u32x2 tr_read(const uint8_t* at) {
+    typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)at));
+}
+
 // Output wave, chunk c (slot S) after the barrier that ends chunk c + 1:
 // o = scale * qg @ hc^T + Aqk @ v_new (kernels.py:268-279).
 // TRAIN: instead of o, store the chunk's hc = bf16(S) as h = hc^T and
 // v_new into the backward's training buffers (blocked by value tile, so a
-// k-tile of this work-group is 512 contiguous bytes), each 16x16 tile
-// quad-transposed to one 8-byte row piece per lane.
-// Two store waves share that work (PART 0: k-tiles 0-3, PART 1: k-tiles
-// 4-7 and v_new); a single wave would fall behind the state wave.
-// WITH_O (a training forward that saves its state): o as well, after the
-// training stores.
-template <int S, bool TRAIN, int PART, bool WITH_O = !TRAIN>
+// k-tile of this work-group is 512 contiguous bytes).  The transposing LDS
+// read does the transpose: lane n of 16 receives as items i = 0..3 the element
+// n % 4 of the 8 bytes that lanes 4*i + n / 4 point at, so with a = n / 4 and
+// those lanes pointing at column 8*(a % 2) + i of k-tile 2*j + a / 2, two reads
+// give each lane 16 bytes of a row, and a store covers both k-tiles (1 KiB).
+// PART 0: k-tiles 0-3, 1: k-tiles 4-7 and v_new, 2: everything (a training
+// forward, whose other output wave forms o; with DPP transposes, 8-byte stores
+// and o behind them in one wave that wave was late: 115 -> 83 us a range of
+// 256 chunks at H = 32, 66 -> 50 us over packed sequences of 4000 tokens).
+template <int S, bool TRAIN, int PART>
 __device__ __forceinline__ void output_step(const Ctx& cx, int c) {
     chunk_barrier();
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (TRAIN) {
-        const int j4 = cx.lane & 3;
         const int cs = cx.rev ? cx.NT - 1 - c : c;  // the chunk of step c
         uint16_t* hrec = cx.trh + (int64_t)cs * TR_H_ELEMS;
 #pragma unroll
-        for (int j = 2 * PART; j < 2 * PART + 2; ++j) {
-            const u32x4 hc = *reinterpret_cast<const u32x4*>(hc_buf[S % HANDOFF] + j * 1024 + cx.lane * 16);
-            const u32x2 t0 = quad_transpose(hc.x, hc.y, j4);
-            const u32x2 t1 = quad_transpose(hc.z, hc.w, j4);
-            const int k0 = 32 * j + 4 * cx.q4 + j4;  // row of k-tile 2j
-            __builtin_nontemporal_store(t0, reinterpret_cast<u32x2*>(hrec + k0 * 16));
-            __builtin_nontemporal_store(t1, reinterpret_cast<u32x2*>(hrec + (k0 + 16) * 16));
+        for (int j = PART == 1 ? 2 : 0; j < (PART == 0 ? 2 : 4); ++j) {
+            const uint8_t* src = hc_buf[S % HANDOFF] + j * 1024 + cx.tr_src;
+            const u32x2 t0 = tr_read(src), t1 = tr_read(src + 64);
+            __builtin_nontemporal_store(u32x4{t0.x, t0.y, t1.x, t1.y}, reinterpret_cast<u32x4*>(hrec + j * 512));
         }
-        if (PART == 1) {
-            const u32x2 vn = *reinterpret_cast<const u32x2*>(vn_buf[S % HANDOFF] + cx.lane * 8);
-            const u32x2 vt = quad_transpose(vn.x, vn.y, j4);
-            __builtin_nontemporal_store(
-                vt, reinterpret_cast<u32x2*>(cx.trvn + (int64_t)cs * TR_VN_ELEMS + (4 * cx.q4 + j4) * 16));
-        }
-        if constexpr (!WITH_O) return;
+        if (PART >= 1)
+            __builtin_nontemporal_store(tr_read(vn_buf[S % HANDOFF] + cx.tr_vsrc),
+                                        reinterpret_cast<u32x2*>(cx.trvn + (int64_t)cs * TR_VN_ELEMS));
+        return;
     }
     const uint8_t* slot = ring + S * SLOT;
     u32x4 hc[4], qg[4];
@@ -477,11 +480,11 @@ __device__ __forceinline__ void state_round_tail(const Ctx& cx, int c, f32x4 (&S
     if constexpr (N > 1) state_round_tail<(S + 1) % RING, N - 1, TPW>(cx, c + 1, St, op, vn);
 }
 
-template <int S, bool TRAIN, int PART, bool WITH_O>
+template <int S, bool TRAIN, int PART>
 __device__ __forceinline__ void output_round(const Ctx& cx, int c) {
-    output_step<S, TRAIN, PART, WITH_O>(cx, c);
+    output_step<S, TRAIN, PART>(cx, c);
     if constexpr (S + 1 < RING) {
-        if (c + 1 < cx.NT) output_round<S + 1, TRAIN, PART, WITH_O>(cx, c + 1);
+        if (c + 1 < cx.NT) output_round<S + 1, TRAIN, PART>(cx, c + 1);
     }
 }
 
@@ -513,24 +516,26 @@ __device__ __forceinline__ void copy_wave(const Params& p, Ctx& cx, const SeqSpa
     copy_barrier();  // the output wave's last chunk
 }
 
-template <bool TRAIN, int PART, bool WITH_O = !TRAIN>
+template <bool TRAIN, int PART>
 __device__ __forceinline__ void output_wave(const Params& p, Ctx& cx, const SeqSpan& sp, int hv) {
     const int x = cx.lane & 15;
-    const int col = 16 * cx.vt + 4 * (x >> 2);
     if constexpr (TRAIN) {
         // forward recompute: h and v_new; backward: dh' and dv_new
         uint16_t* bh = cx.rev ? p.tr_dh : p.tr_h;
         uint16_t* bv = cx.rev ? p.tr_dvn : p.tr_vn;
-        cx.trh = bh + sp.srec0 * TR_H_ELEMS + cx.vt * TR_H_TILE + 4 * (x >> 2);
-        cx.trvn = bv + sp.srec0 * TR_VN_ELEMS + cx.vt * TR_VN_TILE + 4 * (x >> 2);
-    }
-    if constexpr (WITH_O) {
-        cx.obase = p.o + (sp.tok0 * p.HV + hv) * DK + col;
+        const int row = 4 * cx.q4 + (x & 3), a = x >> 2;  // as a destination: the lane's row of a tile
+        cx.trh = bh + sp.srec0 * TR_H_ELEMS + cx.vt * TR_H_TILE + (16 * (a >> 1) + row) * 16 + 8 * (a & 1);
+        cx.trvn = bv + sp.srec0 * TR_VN_ELEMS + cx.vt * TR_VN_TILE + row * 16 + 4 * a;
+        const int i = x >> 2, sa = x & 3;  // as a source: item i of the lanes with a = sa
+        cx.tr_src = (16 * cx.q4 + 8 * (sa & 1) + i) * 16 + 8 * (sa >> 1);
+        cx.tr_vsrc = (16 * cx.q4 + 4 * sa + i) * 8;
+    } else {
+        cx.obase = p.o + (sp.tok0 * p.HV + hv) * DK + 16 * cx.vt + 4 * (x >> 2);
         cx.orow_stride = (int64_t)p.HV * DK;
     }
     chunk_barrier();
     chunk_barrier();
-    for (int c = 0; c < cx.NT; c += RING) output_round<0, TRAIN, PART, WITH_O>(cx, c);
+    for (int c = 0; c < cx.NT; c += RING) output_round<0, TRAIN, PART>(cx, c);
 }
 
 // ---------------------------------------------------------------------------
@@ -548,10 +553,15 @@ __device__ __forceinline__ void output_wave(const Params& p, Ctx& cx, const SeqS
 struct BwdStateOps {
     u32x4 kg[4];
     u32x4 upd[8];
-    u32x2 aqkT;
-    u32x2 dop;
+    u32x4 ad;  // Aqk^T and dO (one member: with two the compiler kept them in LDS)
     f32x2 dc;
 };
+
+__device__ __forceinline__ u32x4 read_ad(const uint8_t* slot, int lane, int vt) {
+    const u32x2 a = *reinterpret_cast<const u32x2*>(slot + BREC_AQKT + lane * 8);
+    const u32x2 d = *reinterpret_cast<const u32x2*>(slot + REC_SHARED + (vt & 1) * 512 + lane * 8);
+    return u32x4{a.x, a.y, d.x, d.y};
+}
 
 __device__ __forceinline__ void read_bwd_ops(const uint8_t* slot, int lane, int vt, BwdStateOps& op) {
 #pragma unroll
@@ -560,27 +570,25 @@ __device__ __forceinline__ void read_bwd_ops(const uint8_t* slot, int lane, int 
 #pragma unroll
     for (int kt = 0; kt < 8; ++kt)
         op.upd[kt] = *reinterpret_cast<const u32x4*>(slot + BREC_UPD + kt * 1024 + lane * 16);
-    op.aqkT = *reinterpret_cast<const u32x2*>(slot + BREC_AQKT + lane * 8);
-    op.dop = *reinterpret_cast<const u32x2*>(slot + REC_SHARED + (vt & 1) * 512 + lane * 8);
+    op.ad = read_ad(slot, lane, vt);
     op.dc = *reinterpret_cast<const f32x2*>(slot + decay_offset(lane));
-}
-
-// dh[kt] = 2^G_last * dh[kt] + upd[kt] @ [dO ; dv_new] for one step's ops.
-template <int KT>
-__device__ __forceinline__ void bwd_update(f32x4 (&D)[8], const BwdStateOps& o, const u32x4& bop) {
-    D[KT] = decay_tile<KT>(D[KT], o.dc);
-    D[KT] = mfma_bf16_16x16x32(as_bf16x8(o.upd[KT]), as_bf16x8(bop), D[KT]);
 }
 
 __device__ __forceinline__ u32x4 pack_tiles(const f32x4& a, const f32x4& b) {
     return u32x4{pack2(a[0], a[1]), pack2(a[2], a[3]), pack2(b[0], b[1]), pack2(b[2], b[3])};
 }
 
-// Step c in slot S, software-pipelined as the forward's state_step: it
-// starts with step c - 1's update, tile by tile, and runs this step's
-// kg @ dh' chain as soon as the tiles it needs are updated.  op[(S+1) & 1]
-// holds step c - 1's operands until its update is done, then receives step
-// c + 1's; bop carries [dO ; dv_new] of step c - 1 in, of step c out.
+// Step c in slot S, laid out as the forward's state_step: it starts with step
+// c - 1's update products, whose decayed dh was formed during that step, and
+// runs this step's kg @ dh' chain as soon as the tiles it needs are updated,
+// with the conversions and this step's decay behind the matrix ops.
+// op[(S+1) & 1] holds step c - 1's operands, each until its update is issued,
+// then receives step c + 1's; bop carries [dO ; dv_new] of step c - 1 in, of
+// step c out.  Without its stores a pass over 512 chunks on 256 work-groups
+// takes 143 us; with decay, product and conversion of a tile pair in one
+// dependent group, and all operands read at the step's end, 259.  With the
+// stores of dh' (537 MB) it is they that bound it: 303 us before and now, and
+// 89 -> 83 us over packed sequences of 4000 tokens, HV = 16.
 template <int S, bool HAS_PREV, bool HAS_NEXT>
 __device__ __forceinline__ void bwd_state_step(const Ctx& cx, f32x4 (&D)[8], BwdStateOps (&op)[2],
                                                u32x4& bop) {
@@ -588,47 +596,82 @@ __device__ __forceinline__ void bwd_state_step(const Ctx& cx, f32x4 (&D)[8], Bwd
     BwdStateOps& oth = op[(S + 1) & 1];
     const uint8_t* ns = ring + ((S + 1) % RING) * SLOT;
     uint8_t* hbuf = hc_buf[S % HANDOFF] + cx.lane * 16;
+    const int lane = cx.lane;
+    auto update = [&](int kt) {  // tile kt of step c - 1's update
+        if (HAS_PREV) D[kt] = mfma_bf16_16x16x32(as_bf16x8(oth.upd[kt]), as_bf16x8(bop), D[kt]);
+    };
+    auto read_kg = [&](int j) {
+        if (HAS_NEXT) oth.kg[j] = *reinterpret_cast<const u32x4*>(ns + BREC_KG + j * 1024 + lane * 16);
+    };
+    auto read_upd = [&](int kt) {
+        if (HAS_NEXT) oth.upd[kt] = *reinterpret_cast<const u32x4*>(ns + BREC_UPD + kt * 1024 + lane * 16);
+    };
+    auto pack_hb = [&](int j) { return pack_tiles(D[2 * j], D[2 * j + 1]); };
+    auto decay = [&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        D[2 * j] = decay_tile<2 * j>(D[2 * j], cur.dc);
+        D[2 * j + 1] = decay_tile<2 * j + 1>(D[2 * j + 1], cur.dc);
+    };
 #define KDA_FENCE() __builtin_amdgcn_sched_barrier(0)
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    update(0);
+    read_kg(0);
+    read_kg(1);
+    KDA_FENCE();
+    update(1);
+    read_kg(2);
+    read_kg(3);
+    KDA_FENCE();
     // Aqk^T dO in the 16x16x32 shape of the chain it starts
-    f32x4 dvn = mfma_bf16_16x16x16_in_x32(cur.aqkT, cur.dop, zero);
-    if (HAS_PREV) {
-        bwd_update<0>(D, oth, bop);
-        bwd_update<1>(D, oth, bop);
+    f32x4 dvn = mfma_bf16_16x16x16_in_x32(u32x2{cur.ad.x, cur.ad.y}, u32x2{cur.ad.z, cur.ad.w}, zero);
+    if (HAS_NEXT) {
+        oth.ad = read_ad(ns, lane, cx.vt);
+        oth.dc = *reinterpret_cast<const f32x2*>(ns + decay_offset(lane));
     }
     KDA_FENCE();
-    const u32x4 hb0 = pack_tiles(D[0], D[1]);
+    update(2);
+    const u32x4 hb0 = pack_hb(0);
+    KDA_FENCE();
+    update(3);
+    decay(std::integral_constant<int, 0>{});
+    KDA_FENCE();
     dvn = mfma_bf16_16x16x32(as_bf16x8(cur.kg[0]), as_bf16x8(hb0), dvn);
-    if (HAS_PREV) {
-        bwd_update<2>(D, oth, bop);
-        bwd_update<3>(D, oth, bop);
-    }
-    *reinterpret_cast<u32x4*>(hbuf + 0 * 1024) = hb0;
+    const u32x4 hb1 = pack_hb(1);
+    read_upd(0);
+    read_upd(1);
     KDA_FENCE();
-    const u32x4 hb1 = pack_tiles(D[2], D[3]);
-    dvn = mfma_bf16_16x16x32(as_bf16x8(cur.kg[1]), as_bf16x8(hb1), dvn);
-    if (HAS_PREV) {
-        bwd_update<4>(D, oth, bop);
-        bwd_update<5>(D, oth, bop);
-    }
+    update(4);
+    decay(std::integral_constant<int, 1>{});
+    KDA_FENCE();
+    update(5);
+    *reinterpret_cast<u32x4*>(hbuf + 0 * 1024) = hb0;
     *reinterpret_cast<u32x4*>(hbuf + 1 * 1024) = hb1;
     KDA_FENCE();
-    const u32x4 hb2 = pack_tiles(D[4], D[5]);
-    dvn = mfma_bf16_16x16x32(as_bf16x8(cur.kg[2]), as_bf16x8(hb2), dvn);
-    if (HAS_PREV) {
-        bwd_update<6>(D, oth, bop);
-        bwd_update<7>(D, oth, bop);
-    }
-    *reinterpret_cast<u32x4*>(hbuf + 2 * 1024) = hb2;
+    dvn = mfma_bf16_16x16x32(as_bf16x8(cur.kg[1]), as_bf16x8(hb1), dvn);
+    read_upd(2);
+    read_upd(3);
     KDA_FENCE();
-    const u32x4 hb3 = pack_tiles(D[6], D[7]);
+    update(6);
+    const u32x4 hb2 = pack_hb(2);
+    KDA_FENCE();
+    update(7);
+    decay(std::integral_constant<int, 2>{});
+    KDA_FENCE();
+    dvn = mfma_bf16_16x16x32(as_bf16x8(cur.kg[2]), as_bf16x8(hb2), dvn);
+    const u32x4 hb3 = pack_hb(3);
+    read_upd(4);
+    read_upd(5);
+    KDA_FENCE();
     dvn = mfma_bf16_16x16x32(as_bf16x8(cur.kg[3]), as_bf16x8(hb3), dvn);
+    decay(std::integral_constant<int, 3>{});
+    *reinterpret_cast<u32x4*>(hbuf + 2 * 1024) = hb2;
     *reinterpret_cast<u32x4*>(hbuf + 3 * 1024) = hb3;
-    if (HAS_NEXT) read_bwd_ops(ns, cx.lane, cx.vt, oth);
+    read_upd(6);
+    read_upd(7);
     KDA_FENCE();
     const u32x2 dvb = {pack2(dvn[0], dvn[1]), pack2(dvn[2], dvn[3])};
-    *reinterpret_cast<u32x2*>(vn_buf[S % HANDOFF] + cx.lane * 8) = dvb;
-    bop = u32x4{cur.dop.x, cur.dop.y, dvb.x, dvb.y};
+    *reinterpret_cast<u32x2*>(vn_buf[S % HANDOFF] + lane * 8) = dvb;
+    bop = u32x4{cur.ad.z, cur.ad.w, dvb.x, dvb.y};
     if (HAS_NEXT) {
         chunk_barrier_nodrain();
     } else {
@@ -637,14 +680,9 @@ __device__ __forceinline__ void bwd_state_step(const Ctx& cx, f32x4 (&D)[8], Bwd
     KDA_FENCE();
     if (!HAS_NEXT) {
         // the last step's update: dh becomes the initial state's gradient
-        bwd_update<0>(D, cur, bop);
-        bwd_update<1>(D, cur, bop);
-        bwd_update<2>(D, cur, bop);
-        bwd_update<3>(D, cur, bop);
-        bwd_update<4>(D, cur, bop);
-        bwd_update<5>(D, cur, bop);
-        bwd_update<6>(D, cur, bop);
-        bwd_update<7>(D, cur, bop);
+#pragma unroll
+        for (int kt = 0; kt < 8; ++kt)
+            D[kt] = mfma_bf16_16x16x32(as_bf16x8(cur.upd[kt]), as_bf16x8(bop), D[kt]);
     }
 #undef KDA_FENCE
 }
@@ -1061,8 +1099,8 @@ enum Role { STATE = 0, OUTPUT = 1, COPY = 2, OUTPUT2 = 3 };
 // MODE K2_FWD_MS: the forward with several sequences per work-group
 // (above); grid seq_groups * HV * 8.  MODE K2_TRAIN_O: a training forward
 // that keeps its state for the backward: o and ht as K2_FWD (the same
-// arithmetic, so bit for bit), and h and v_new as K2_TRAIN; the first
-// store wave forms o.
+// arithmetic, so bit for bit), and h and v_new as K2_TRAIN; the output
+// wave forms o and OUTPUT2 stores the rest.
 enum K2Mode { K2_FWD = 0, K2_TRAIN = 1, K2_BWD = 2, K2_FWD_MS = 3, K2_TRAIN_O = 4 };
 
 // The training modes run a fourth wave, OUTPUT2, the second store wave.
@@ -1144,12 +1182,12 @@ __global__ __launch_bounds__(MODE == K2_FWD || MODE == K2_FWD_MS ? 192 : 256) vo
         __builtin_amdgcn_endpgm();
     }
     if (role == OUTPUT) {
-        output_wave<STORE_TR, 0, !STORE_TR || MODE == K2_TRAIN_O>(p, cx, sp, hv);
+        output_wave<STORE_TR && MODE != K2_TRAIN_O, 0>(p, cx, sp, hv);
         __builtin_amdgcn_endpgm();
     }
     if constexpr (STORE_TR) {
         if (role == OUTPUT2) {
-            output_wave<STORE_TR, 1, false>(p, cx, sp, hv);
+            output_wave<true, MODE == K2_TRAIN_O ? 2 : 1>(p, cx, sp, hv);
             __builtin_amdgcn_endpgm();
         }
     }
