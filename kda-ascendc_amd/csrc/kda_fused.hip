@@ -382,7 +382,8 @@ __global__ __launch_bounds__(F_THREADS) void fused_kernel(Params p) {
 
 // Estimated times (us) of a varlen forward on `ncu` CUs, from per-chunk
 // costs measured on MI355X (K = V = 128, every in-kernel flag):
-//   fused: each work-group takes ~1.85 us per chunk of its sequence, in
+//   fused: each work-group takes ~1.85 us per chunk of its sequence (1.74
+//   since it has eight producers; the line was measured at 1.85), in
 //     parallel with the others, so the longest sequence sets the time, or
 //     the chunks per CU once the work-groups run in rounds;
 //   two stages: stage 1 ~7.5 ns per record slot and value head, stage 2
@@ -411,7 +412,7 @@ double two_stage_estimate_us(const Params& p, int ncu) {
 // when the pairs fill the CUs.
 //
 // Below the CU count the fused kernel runs every pair in one round of
-// work-groups, about 1.85 us per chunk whatever their number, while the two
+// work-groups, about 1.74 us per chunk whatever their number, while the two
 // stages grow with the pairs (T=4096 forwards, two stages against fused: 128
 // pairs 377 against 476 us, 160 pairs 505 against 480, 224 pairs 658 against
 // 479).  With cu_seqlens the fused kernel's time follows the longest
