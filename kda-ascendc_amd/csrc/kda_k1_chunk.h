@@ -309,13 +309,17 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
     f32x4 acc_qk = {0.f, 0.f, 0.f, 0.f};
     f32x4 acc_kk = {0.f, 0.f, 0.f, 0.f};
     // One pass over the columns forms everything that needs the gates: the
-    // grams' operands; kg = bf16(k^ * 2^(G_last - G)) (kernels.py:282-290) as
-    // the gram's k^ * 2^(G_mid - G) times row last's 2^(G_last - G_mid); kb =
-    // bf16(bf16(k^ * beta) * 2^G) (kernels.py:171); and qg = bf16(q^ * 2^G),
-    // the gated query stage 2 multiplies the state by (kernels.py:269).  kb
-    // and kg go to LDS tiles, to be read back in T order.  q^, k^ and G are
-    // unpacked and read once and die here, which leaves the rest of the chunk
-    // 122 registers where separate passes held 160.
+    // grams' operands; kg = bf16(k^ * 2^(G_last - G)) (kernels.py:282-290);
+    // kb = bf16(bf16(k^ * beta) * 2^G) (kernels.py:171); and qg =
+    // bf16(q^ * 2^G), the gated query stage 2 multiplies the state by
+    // (kernels.py:269).  kb and kg go to LDS tiles, to be read back in T
+    // order.  q^, k^ and G are unpacked and read once and die here, which
+    // leaves the rest of the chunk 122 registers where separate passes held
+    // 160.  kg's exponential is its own, of an argument that is never
+    // positive: the product of the grams' 2^(G_mid - G) and 2^(G_last - G_mid)
+    // leaves the fp32 range where a token's decay is below 2^-126, and there
+    // the state after it was lost (B=16 T=2048 H=32, fused: 443 us with the
+    // product, 453 without).
     hk.slot();
     u32x2 kgF[8], qgp[8];
     bcast_mid([&](auto from_mid) {
@@ -335,7 +339,7 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
                     // receives Aqk[t][4*q4 + i] and Akk[t][4*q4 + i].
                     acc_qk = mfma_f32_16x16x4(ks, qv * gq, acc_qk);
                     acc_kk = mfma_f32_16x16x4(ks, kv * gq, acc_kk);
-                    kg[i] = ks * from_last(gq);
+                    kg[i] = kv * fast_exp2(from_last(G[j]) - G[j]);
                     e[i] = fast_exp2(G[j]);
                     kb[i] = kv * beta;
                     qg[i] = qv * e[i];
