@@ -310,11 +310,13 @@ __global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(2))) void bw
         }
         sq2 = row_sum16(sq2);
         sk2 = row_sum16(sk2);
-        rq = 1.f / sqrtf(sq2 + L2_EPS);
-        rk = 1.f / sqrtf(sk2 + L2_EPS);
+        rq = inv_norm(sq2);
+        rk = inv_norm(sk2);
     }
-    // q^ and k^ as the forward rounds them (bf16 after the l2norm)
-    // (zero in rows past the last token)
+    // q^ and k^ as the forward rounds them (bf16 after the l2norm; the squares
+    // are added in this kernel's order, so where that moves the norm's last bit
+    // an element at a rounding boundary is the neighbouring bf16), zero in rows
+    // past the last token
     auto qk_hat = [&](float (&qn)[8], float (&kn)[8]) {
         unpack8(qraw, qn);
         unpack8(kraw, kn);

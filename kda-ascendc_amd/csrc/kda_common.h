@@ -284,10 +284,9 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
 __device__ __forceinline__ float lo_f(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
 __device__ __forceinline__ float hi_f(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
 
-// c + a.lo * b.lo + a.hi * b.hi in fp32, a and b two bf16 each.
-__device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), c, false);
-}
+// The l2norm's factor 1 / sqrt(sum + eps) (kernels.py:108-113), root and
+// quotient correctly rounded, for the forward and the backward alike.
+__device__ __forceinline__ float inv_norm(float sum) { return 1.f / sqrtf(sum + L2_EPS); }
 
 // exp2 on the transcendental unit (v_exp_f32, 1 ulp), without the library
 // routine's denormal-range fixups: every exponent that reaches it is either

@@ -244,26 +244,27 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
     if (p.use_beta_sigmoid) beta = fast_sigmoid(beta);
 
     // ---- q/k l2norm, rounded back to bf16 (kernels.py:108-113) -----------
+    // The sum is a chain of fused multiply-adds per lane (the two-term dot
+    // instruction rounds otherwise).  Outside the fused forward the row passes
+    // through an opaque statement and is unpacked again for the products:
+    // held unpacked it takes stage 1 from four waves per SIMD to three.
     if (p.use_l2norm) {
-        float sq = 0.f, sk = 0.f;
+        auto unit = [&](Row32& x) {
+            float s = 0.f;
 #pragma unroll
-        for (int kt = 0; kt < 8; ++kt) {
-            sq = dot2(qp.v[kt].y, qp.v[kt].y, dot2(qp.v[kt].x, qp.v[kt].x, sq));
-            sk = dot2(kp.v[kt].y, kp.v[kt].y, dot2(kp.v[kt].x, kp.v[kt].x, sk));
-        }
-        sq += xor16(sq);
-        sk += xor16(sk);
-        sq += __shfl_xor(sq, 32);
-        sk += __shfl_xor(sk, 32);
-        const float rq = __builtin_amdgcn_rsqf(sq + L2_EPS);
-        const float rk = __builtin_amdgcn_rsqf(sk + L2_EPS);
+            for (int j = 0; j < 32; ++j) s = fmaf(elem(x, j), elem(x, j), s);
+            s += xor16(s);
+            s += __shfl_xor(s, 32);
+            const float rn = inv_norm(s);
 #pragma unroll
-        for (int kt = 0; kt < 8; ++kt) {
-            qp.v[kt] = pack4(elem(qp, 4 * kt) * rq, elem(qp, 4 * kt + 1) * rq,
-                             elem(qp, 4 * kt + 2) * rq, elem(qp, 4 * kt + 3) * rq);
-            kp.v[kt] = pack4(elem(kp, 4 * kt) * rk, elem(kp, 4 * kt + 1) * rk,
-                             elem(kp, 4 * kt + 2) * rk, elem(kp, 4 * kt + 3) * rk);
-        }
+            for (int kt = 0; kt < 8; ++kt) {
+                if constexpr (!U_IN_SLOT) asm("" : "+v"(x.v[kt].x), "+v"(x.v[kt].y));
+                x.v[kt] = pack4(elem(x, 4 * kt) * rn, elem(x, 4 * kt + 1) * rn,
+                                elem(x, 4 * kt + 2) * rn, elem(x, 4 * kt + 3) * rn);
+            }
+        };
+        unit(qp);
+        unit(kp);
     }
 
     // ---- gate and chunk-local log2 cumsum (kernels.py:115-124) -----------
