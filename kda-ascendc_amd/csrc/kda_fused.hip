@@ -265,7 +265,7 @@ __device__ __forceinline__ void produce(const Params& p, int h, int hv, int c, c
     // A_inv and beta go after it
     const K1Scratch scr{f_L[s], reinterpret_cast<float*>(rec + FREC_A), rec + REC_W, rec + REC_KG};
     const ProducerHooks<FULL, GB16> hk{p, sp, in, h, hv, c, lane};
-    k1_compute<K1_FWD, FULL, GB16, true>(p, hv, c, sp, in, f_bias, ea, scr, rec, hk);
+    k1_compute<K1_FWD, FULL, GB16, true, true>(p, hv, c, sp, in, f_bias, ea, scr, rec, hk);
     // the record's LDS writes have completed before the slot is marked full
     // (v's rows had landed before tail() went on)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

@@ -22,20 +22,16 @@ namespace kda {
 
 namespace {
 
-// The forward's records: 122-129 VGPRs and 10 KiB of LDS a wave, so four waves
-// per SIMD (three with fp32 g and partial chunks).  A wave spends most of its
-// life waiting on memory, which sets the time (4.6 TB/s of a copy's 5.2);
-// held to three waves per SIMD B=2 T=4096 H=8 takes 100 against 96 us.
+// A wave spends most of its life waiting on memory (16.4 KiB read and 17 KiB
+// written a chunk; 4.6 TB/s of a copy's 5.2 at T=8192 H=32).  The forward's
+// records take 160-166 VGPRs, three waves per SIMD, or in one pass 122-125
+// and 10 KiB of LDS, four waves (forward_in_one_pass).
 //
 // K1M (the record modes, below) other than K1_FWD also writes the backward
 // record (kda_common.h) to p.ws_bwd: the same chunk quantities in the
 // operand orders of the reverse state chain, from one read of the inputs,
 // and the gram block to p.la.  Those modes hold more: K1_SAVE runs three
 // waves per SIMD, K1_BOTH two.
-// LDS of a work-group (one wave): k1_chunk's scratch.
-__shared__ __attribute__((aligned(16))) float s_L[BT * BT];
-__shared__ float s_X[BT * BT];
-__shared__ __attribute__((aligned(16))) uint8_t s_kb[TILE_BYTES], s_kg[TILE_BYTES];
 
 // The (value head, chunk, sequence) of this work-group; false for a gap
 // slot (wave-uniform, before any barrier).  With cu_seqlens, slot x of
@@ -65,13 +61,22 @@ __device__ __forceinline__ bool block_chunk(const Params& p, int lane, int& hv, 
 // ALL_FULL: fixed-length batch with T a multiple of 16, so every chunk is
 // full.  Otherwise every chunk takes the general path: both variants in one
 // kernel would not fit the register budget of three waves per SIMD.
-template <int K1M, bool ALL_FULL, bool GB16>
+template <int K1M, bool ALL_FULL, bool GB16, bool ONE_PASS>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(K1M != K1_FWD ? 2 : 3))) void k1_kernel(Params p) {
     int hv, c;
     SeqSpan sp;
     if (!block_chunk(p, threadIdx.x, hv, c, sp)) return;
-    k1_chunk<K1M, ALL_FULL, GB16>(p, hv, c, sp, K1Scratch{s_L, s_X, s_kb, s_kg}, p.ws + (sp.rec0 + c) * REC_BYTES);
+    // a wave's scratch: 10 KiB in one pass, so that sixteen waves fit a CU
+    __shared__ __attribute__((aligned(16))) float s_L[BT * BT];
+    __shared__ float s_X[ONE_PASS ? BT * BT : BT * (BT + 1)];
+    K1Scratch scr{s_L, s_X, nullptr, nullptr};
+    if constexpr (ONE_PASS) {
+        __shared__ __attribute__((aligned(16))) uint8_t s_tiles[2 * TILE_BYTES];
+        scr.kb = s_tiles;
+        scr.kg = s_tiles + TILE_BYTES;
+    }
+    k1_chunk<K1M, ALL_FULL, GB16, ONE_PASS>(p, hv, c, sp, scr, p.ws + (sp.rec0 + c) * REC_BYTES);
 }
 
 // The dO operand of each backward record that a training forward saved
@@ -103,21 +108,47 @@ int64_t k1_grid(const Params& p) {
     return p.cu_seqlens ? (int64_t)p.HV * p.NS : (int64_t)p.B * p.HV * p.NT;
 }
 
-template <int K1M>
+template <int K1M, bool ONE_PASS>
 hipError_t launch(const Params& p, hipStream_t stream) {
     const bool all_full = !p.cu_seqlens && p.T % BT == 0;
-    auto kern = all_full ? (p.g_bf16 ? k1_kernel<K1M, true, true> : k1_kernel<K1M, true, false>)
-                         : (p.g_bf16 ? k1_kernel<K1M, false, true> : k1_kernel<K1M, false, false>);
+    auto kern = all_full ? k1_kernel<K1M, true, true, ONE_PASS> : k1_kernel<K1M, false, true, ONE_PASS>;
+    // (fp32 g in one pass takes more than the registers of four waves per SIMD)
+    if constexpr (!ONE_PASS || K1M != K1_FWD) {
+        if (!p.g_bf16) kern = all_full ? k1_kernel<K1M, true, false, ONE_PASS> : k1_kernel<K1M, false, false, ONE_PASS>;
+    }
     hipLaunchKernelGGL(kern, dim3((unsigned)k1_grid(p)), dim3(64), 0, stream, p);
     return hipGetLastError();
 }
 }  // namespace
 
-hipError_t launch_k1(const Params& p, hipStream_t stream) { return launch<K1_FWD>(p, stream); }
+// Whether the forward's records are formed in one pass over the columns
+// (k1_compute).  Its registers allow four waves per SIMD, so the card's 1024
+// SIMDs hold 4096 chunks at once where passes of their own hold 3072; in turn
+// it stores with the LDS tiles' round trips in between, which the small
+// launches feel as latency and the large ones, bound by their stores, as 1.5 %.
+// The partial-chunk code issues a fifth more, and gains the more.  Us, one pass
+// against passes of their own, by chunks:
+//   whole chunks: 3072 24.5 / 23.4, 3584 28.8 / 28.6, 4096 29.9 / 30.1, 5120
+//     35.2 / 36.6, 7168 48.8 / 50.0, 8192 60.9 / 59.6, 12288 (H=48) 95 / 92;
+//   partial ones: 3072 27.7 / 27.2, 3200 30.8 / 31.4, 4096 32.1 / 34.6, 8192
+//     60.6 / 64.8, 9216 69.8 / 70.3, 10240 81.8 / 79.0;
+//   packed sequences: 2000 (H=16) 25.8 / 25.6, 4000 32.6 / 36.0, 8100 61.3 /
+//     67.6, 16400 115.8 / 119.1, 33000 228.4 / 229.7.
+// fp32 g holds too much for four waves and never gains.
+static bool forward_in_one_pass(const Params& p) {
+    const int64_t chunks = k1_grid(p);
+    if (!p.g_bf16 || chunks <= 3072) return false;
+    if (p.cu_seqlens) return true;
+    return p.T % BT == 0 ? chunks > 3840 && chunks <= 7168 : chunks <= 9216;
+}
 
-hipError_t launch_k1_both_records(const Params& p, hipStream_t stream) { return launch<K1_BOTH>(p, stream); }
+hipError_t launch_k1(const Params& p, hipStream_t stream) {
+    return forward_in_one_pass(p) ? launch<K1_FWD, true>(p, stream) : launch<K1_FWD, false>(p, stream);
+}
 
-hipError_t launch_k1_save(const Params& p, hipStream_t stream) { return launch<K1_SAVE>(p, stream); }
+hipError_t launch_k1_both_records(const Params& p, hipStream_t stream) { return launch<K1_BOTH, true>(p, stream); }
+
+hipError_t launch_k1_save(const Params& p, hipStream_t stream) { return launch<K1_SAVE, true>(p, stream); }
 
 hipError_t launch_k1_dout(const Params& p, hipStream_t stream) {
     hipLaunchKernelGGL(k1_dout_kernel, dim3((unsigned)k1_grid(p)), dim3(64), 0, stream, p);

@@ -89,8 +89,8 @@ __device__ __forceinline__ u32x2 form_u(i16x4 vbT, i16x4 A_op) {
 // and the tile buffers of kb and kg.
 struct K1Scratch {
     float* L;     // [16][16]
-    float* X;     // [16][16], column s at 16 * s, element t at t ^ s of it
-    uint8_t* kb;  // TILE_BYTES
+    float* X;     // in one pass [16][16], column s at 16 * s, element t at t ^ s of it; else column s at 17 * s
+    uint8_t* kb;  // TILE_BYTES (the tiles in one pass only)
     uint8_t* kg;  // TILE_BYTES
 };
 
@@ -205,11 +205,20 @@ struct K1NoHooks {
 // The work on one chunk's inputs: biasp the head's dt_bias (k1_bias, or a
 // copy of it), ea = k1_ea.  U_IN_SLOT: `rec` is a ring slot of the fused
 // forward (FREC_*); v is not touched here.
-template <int K1M, bool FULL, bool GB16, bool U_IN_SLOT = false, class Hooks = K1NoHooks>
+//
+// ONE_PASS: one pass over the columns forms everything that needs the gates,
+// and operands change order through LDS tiles: fewer registers and matrix ops,
+// for the fused forward's producers, the training modes and some forwards.
+// Without it the grams, w's and qg's operands and kg are formed in passes of
+// their own, transposed by the matrix core and stored as they are formed, which
+// is the shorter where latency or the stores bind (forward_in_one_pass,
+// kda_k1.hip).  The two give the same bits.
+template <int K1M, bool FULL, bool GB16, bool ONE_PASS, bool U_IN_SLOT = false, class Hooks = K1NoHooks>
 __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const SeqSpan& sp,
                                            const K1In<GB16, K1M == K1_BOTH>& in, const float* biasp,
                                            float ea, const K1Scratch& scr, uint8_t* rec,
                                            Hooks hk = Hooks{}) {
+    static_assert(ONE_PASS || (K1M == K1_FWD && !U_IN_SLOT), "the passes of their own form the forward record only");
     constexpr bool BOTH = K1M != K1_FWD;
     constexpr bool WITH_DO = K1M == K1_BOTH;
     const K1Row w = k1_row<FULL>(p, hv, c, sp);
@@ -245,26 +254,31 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
 
     // ---- q/k l2norm, rounded back to bf16 (kernels.py:108-113) -----------
     // The sum is a chain of fused multiply-adds per lane (the two-term dot
-    // instruction rounds otherwise).  Outside the fused forward the row passes
-    // through an opaque statement and is unpacked again for the products:
-    // held unpacked it takes stage 1 from four waves per SIMD to three.
+    // instruction rounds otherwise).  In one pass outside the fused forward the
+    // row goes through an opaque statement and is unpacked again for the
+    // products: held unpacked it takes four waves per SIMD to three.
     if (p.use_l2norm) {
-        auto unit = [&](Row32& x) {
-            float s = 0.f;
+        float sq = 0.f, sk = 0.f;
 #pragma unroll
-            for (int j = 0; j < 32; ++j) s = fmaf(elem(x, j), elem(x, j), s);
-            s += xor16(s);
-            s += __shfl_xor(s, 32);
-            const float rn = inv_norm(s);
+        for (int j = 0; j < 32; ++j) {
+            sq = fmaf(elem(qp, j), elem(qp, j), sq);
+            sk = fmaf(elem(kp, j), elem(kp, j), sk);
+        }
+        sq += xor16(sq);
+        sk += xor16(sk);
+        sq += __shfl_xor(sq, 32);
+        sk += __shfl_xor(sk, 32);
+        const float rq = inv_norm(sq), rk = inv_norm(sk);
+        auto times = [&](Row32& x, float rn) {
 #pragma unroll
             for (int kt = 0; kt < 8; ++kt) {
-                if constexpr (!U_IN_SLOT) asm("" : "+v"(x.v[kt].x), "+v"(x.v[kt].y));
+                if constexpr (ONE_PASS && !U_IN_SLOT) asm("" : "+v"(x.v[kt].x), "+v"(x.v[kt].y));
                 x.v[kt] = pack4(elem(x, 4 * kt) * rn, elem(x, 4 * kt + 1) * rn,
                                 elem(x, 4 * kt + 2) * rn, elem(x, 4 * kt + 3) * rn);
             }
         };
-        unit(qp);
-        unit(kp);
+        times(qp, rq);
+        times(kp, rk);
     }
 
     // ---- gate and chunk-local log2 cumsum (kernels.py:115-124) -----------
@@ -309,60 +323,76 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
     };
     f32x4 acc_qk = {0.f, 0.f, 0.f, 0.f};
     f32x4 acc_kk = {0.f, 0.f, 0.f, 0.f};
-    // One pass over the columns forms everything that needs the gates: the
-    // grams' operands; kg = bf16(k^ * 2^(G_last - G)) (kernels.py:282-290);
-    // kb = bf16(bf16(k^ * beta) * 2^G) (kernels.py:171); and qg =
-    // bf16(q^ * 2^G), the gated query stage 2 multiplies the state by
-    // (kernels.py:269).  kb and kg go to LDS tiles, to be read back in T
-    // order.  q^, k^ and G are unpacked and read once and die here, which
-    // leaves the rest of the chunk 122 registers where separate passes held
-    // 160.  kg's exponential is its own, of an argument that is never
-    // positive: the product of the grams' 2^(G_mid - G) and 2^(G_last - G_mid)
-    // leaves the fp32 range where a token's decay is below 2^-126, and there
-    // the state after it was lost (B=16 T=2048 H=32, fused: 443 us with the
-    // product, 453 without).
+    // kg = bf16(k^ * 2^(G_last - G)) (kernels.py:282-290); kb =
+    // bf16(bf16(k^ * beta) * 2^G) (kernels.py:171); and qg = bf16(q^ * 2^G),
+    // the gated query stage 2 multiplies the state by (kernels.py:269).  kg's
+    // exponential is its own, of an argument that is never positive: the
+    // product of the grams' 2^(G_mid - G) and 2^(G_last - G_mid) leaves the
+    // fp32 range where a token's decay is below 2^-126, and there the state
+    // after it was lost (B=16 T=2048 H=32, fused: 443 us with the product, 453
+    // without).  In one pass kb and kg go to LDS tiles, to be read back in T
+    // order, and q^, k^ and G are unpacked and read once and die here.
     hk.slot();
     u32x2 kgF[8], qgp[8];
-    bcast_mid([&](auto from_mid) {
-        bcast_last([&](auto from_last) {
+    // Columns 4*kt + i of both grams; A = Ks (rows s), B = Qs / Kq (columns t):
+    // lane (t, q4) receives Aqk[t][4*q4 + i] and Akk[t][4*q4 + i].
+    auto gram = [&](int j, float qv, float kv, auto from_mid) {
+        const float gm = G[j] - from_mid(G[j]);
+        const float gq = valid ? fast_exp2(gm) : 0.f;
+        const float gk = valid ? fast_exp2(-gm) : 0.f;
+        acc_qk = mfma_f32_16x16x4(kv * gk, qv * gq, acc_qk);
+        acc_kk = mfma_f32_16x16x4(kv * gk, kv * gq, acc_kk);
+    };
+    // e[i] = 2^G, and kb and qg of tile kt; the state's decay 2^G_last
+    // (kernels.py:282-290) is 2^G on the chunk's last row.
+    auto gated = [&](int kt, u32x2& kb, u32x2& qg) {
+        float e[4], kbv[4], qgv[4];
 #pragma unroll
-            for (int kt = 0; kt < 8; ++kt) {
-                float kg[4], kb[4], qg[4], e[4];
+        for (int i = 0; i < 4; ++i) {
+            e[i] = fast_exp2(G[4 * kt + i]);
+            kbv[i] = elem(kp, 4 * kt + i) * beta;
+            qgv[i] = elem(qp, 4 * kt + i) * e[i];
+        }
+        const u32x2 kbr = pack4(kbv[0], kbv[1], kbv[2], kbv[3]);
+        kb = pack4(lo_f(kbr.x) * e[0], hi_f(kbr.x) * e[1], lo_f(kbr.y) * e[2], hi_f(kbr.y) * e[3]);
+        qg = pack4(qgv[0], qgv[1], qgv[2], qgv[3]);
+        if (r == last)
+            *reinterpret_cast<f32x4*>(rec + REC_DECAY + kt * 64 + q4 * 16) = f32x4{e[0], e[1], e[2], e[3]};
+    };
+    auto kg_tile = [&](int kt, auto from_last) {
+        float kg[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int j = 4 * kt + i;
-                    const float gm = G[j] - from_mid(G[j]);
-                    const float gq = valid ? fast_exp2(gm) : 0.f;
-                    const float gk = valid ? fast_exp2(-gm) : 0.f;
-                    const float qv = elem(qp, j), kv = elem(kp, j);
-                    const float ks = kv * gk;
-                    // A = Ks (rows s), B = Qs / Kq (columns t): lane (t, q4)
-                    // receives Aqk[t][4*q4 + i] and Akk[t][4*q4 + i].
-                    acc_qk = mfma_f32_16x16x4(ks, qv * gq, acc_qk);
-                    acc_kk = mfma_f32_16x16x4(ks, kv * gq, acc_kk);
-                    kg[i] = kv * fast_exp2(from_last(G[j]) - G[j]);
-                    e[i] = fast_exp2(G[j]);
-                    kb[i] = kv * beta;
-                    qg[i] = qv * e[i];
+        for (int i = 0; i < 4; ++i)
+            kg[i] = elem(kp, 4 * kt + i) * fast_exp2(from_last(G[4 * kt + i]) - G[4 * kt + i]);
+        return pack4(kg[0], kg[1], kg[2], kg[3]);
+    };
+    auto store_pair = [&](int at, int j, u32x2 a, u32x2 b) {
+        *reinterpret_cast<u32x4*>(rec + at + j * 1024 + lane * 16) = u32x4{a.x, a.y, b.x, b.y};
+    };
+    if constexpr (ONE_PASS) {
+        bcast_mid([&](auto from_mid) {
+            bcast_last([&](auto from_last) {
+#pragma unroll
+                for (int kt = 0; kt < 8; ++kt) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        gram(4 * kt + i, elem(qp, 4 * kt + i), elem(kp, 4 * kt + i), from_mid);
+                    u32x2 kb;
+                    gated(kt, kb, qgp[kt]);
+                    put_F(scr.kb, kt, lane, kb);
+                    kgF[kt] = kg_tile(kt, from_last);
+                    put_F(scr.kg, kt, lane, kgF[kt]);
+                    // (the backward's recompute produces no o and never reads qg)
+                    if (K1M != K1_BOTH && (kt & 1)) store_pair(REC_QG, kt >> 1, qgp[kt - 1], qgp[kt]);
                 }
-                const u32x2 kbr = pack4(kb[0], kb[1], kb[2], kb[3]);
-                const u32x2 kbe = pack4(lo_f(kbr.x) * e[0], hi_f(kbr.x) * e[1],
-                                        lo_f(kbr.y) * e[2], hi_f(kbr.y) * e[3]);
-                put_F(scr.kb, kt, lane, kbe);
-                kgF[kt] = pack4(kg[0], kg[1], kg[2], kg[3]);
-                put_F(scr.kg, kt, lane, kgF[kt]);
-                // the state's decay 2^G_last (kernels.py:282-290): on the
-                // chunk's last row, 2^G is it
-                if (r == last)
-                    *reinterpret_cast<f32x4*>(rec + REC_DECAY + kt * 64 + q4 * 16) = f32x4{e[0], e[1], e[2], e[3]};
-                qgp[kt] = pack4(qg[0], qg[1], qg[2], qg[3]);
-                // (the backward's recompute produces no o and never reads qg)
-                if (K1M != K1_BOTH && (kt & 1))
-                    *reinterpret_cast<u32x4*>(rec + REC_QG + (kt >> 1) * 1024 + lane * 16) =
-                        u32x4{qgp[kt - 1].x, qgp[kt - 1].y, qgp[kt].x, qgp[kt].y};
-            }
+            });
         });
-    });
+    } else {
+        bcast_mid([&](auto from_mid) {
+#pragma unroll
+            for (int j = 0; j < 32; ++j) gram(j, elem(qp, j), elem(kp, j), from_mid);
+        });
+    }
 
     // This chunk's record goes to `rec` with ordinary stores: in the
     // workspace, the grid runs the chunks last to first (k1_kernel), so the
@@ -387,6 +417,7 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
     // a[t < s] = 0 and a[t > s] = -sum_{j<t} L[t][j] a[j].
     *reinterpret_cast<f32x4*>(scr.L + r * BT + 4 * q4) = L;
     wave_lds_fence();
+    auto x_at = [](int s, int t) { return ONE_PASS ? BT * s + (t ^ s) : (BT + 1) * s + t; };
     {
         float a[BT];
 #pragma unroll
@@ -406,13 +437,13 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
         }
         if (q4 == 0) {
 #pragma unroll
-            for (int t = 0; t < BT; ++t) scr.X[r * BT + (t ^ r)] = a[t];
+            for (int t = 0; t < BT; ++t) scr.X[x_at(r, t)] = a[t];
         }
     }
     wave_lds_fence();
     f32x4 ainv;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) ainv[i] = scr.X[(4 * q4 + i) * BT + (r ^ (4 * q4 + i))];
+    for (int i = 0; i < 4; ++i) ainv[i] = scr.X[x_at(4 * q4 + i, r)];
     const u32x2 ainv_bf = pack4(ainv);  // A = bf16(A_inv), kernels.py:170
     if constexpr (BOTH) {
         // the gram and the inverse for the per-chunk gradients (kda_common.h)
@@ -425,8 +456,50 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
     // the identity operand of the transposes through the matrix core (tile_T)
     const i16x4 eye = eye_operand(lane);
     i16x4 kbT[8];
+    if constexpr (ONE_PASS) {
 #pragma unroll
-    for (int kt = 0; kt < 8; ++kt) kbT[kt] = get_T(scr.kb, kt, lane);
+        for (int kt = 0; kt < 8; ++kt) kbT[kt] = get_T(scr.kb, kt, lane);
+    }
+
+    // ---- u = A @ bf16(v * beta) (kernels.py:173-174) ----------------------
+    // One 16x16x16 tile per 16 value columns; u lands as
+    // u[4*q4 + i][16*vt + r], the order stage 2 subtracts it in.  (In the
+    // fused forward's slot the operands go in u's place instead: FREC_*,
+    // below.)
+    if constexpr (!U_IN_SLOT) {
+        auto vb = [&](int vt) {
+            return pack4(elem(vp, 4 * vt) * beta, elem(vp, 4 * vt + 1) * beta,
+                         elem(vp, 4 * vt + 2) * beta, elem(vp, 4 * vt + 3) * beta);
+        };
+        if constexpr (ONE_PASS) {
+#pragma unroll
+            for (int vt = 0; vt < 8; ++vt) put_F(scr.kb, vt, lane, vb(vt));
+            wave_lds_fence();
+        }
+#pragma unroll
+        for (int vt = 0; vt < 8; ++vt) {
+            const u32x2 ub = form_u(ONE_PASS ? get_T(scr.kb, vt, lane) : tile_T(vb(vt), eye), A_op);
+            *reinterpret_cast<u32x2*>(rec + REC_U + vt * 512 + lane * 8) = ub;
+            if (p.dbg_u) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int row = 4 * q4 + i;
+                    if (row < nvalid) {
+                        const int64_t o = ((sp.tok0 + t0 + row) * HV + hv) * DK + 16 * vt + r;
+                        p.dbg_u[o] = (uint16_t)(i == 0 ? ub.x : i == 1 ? (ub.x >> 16)
+                                                : i == 2 ? ub.y : (ub.y >> 16));
+                    }
+                }
+            }
+        }
+    }
+    u32x2 kbF[8];
+    if constexpr (!ONE_PASS) {
+#pragma unroll
+        for (int kt = 0; kt < 8; ++kt) gated(kt, kbF[kt], qgp[kt]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) store_pair(REC_QG, j, qgp[2 * j], qgp[2 * j + 1]);
+    }
 
     if constexpr (BOTH) {
         // ---- backward record ---------------------------------------------
@@ -489,50 +562,24 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
 #pragma unroll
     for (int kt = 0; kt < 8; ++kt) {
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-        wpk[kt] = pack4(mfma_bf16_16x16x16(kbT[kt], A_neg, zero));
+        wpk[kt] = pack4(mfma_bf16_16x16x16(ONE_PASS ? kbT[kt] : tile_T(kbF[kt], eye), A_neg, zero));
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const u32x4 wj = {wpk[2 * j].x, wpk[2 * j].y, wpk[2 * j + 1].x, wpk[2 * j + 1].y};
-        *reinterpret_cast<u32x4*>(rec + REC_W + j * 1024 + lane * 16) = wj;
-    }
+    for (int j = 0; j < 4; ++j) store_pair(REC_W, j, wpk[2 * j], wpk[2 * j + 1]);
 
-    // ---- u = A @ bf16(v * beta) (kernels.py:173-174) ----------------------
-    // One 16x16x16 tile per 16 value columns; u lands as
-    // u[4*q4 + i][16*vt + r], the order stage 2 subtracts it in.  In the
-    // fused forward's slot the operands go in u's place instead (FREC_*).
-    // kg goes out in T order (stage 2's A operand), or stays as tiles there.
+    // kg goes out in T order (stage 2's A operand); in the fused forward's slot
+    // it stays as tiles, and bf16(A_inv) and beta follow the raw v.
     if constexpr (U_IN_SLOT) {
         *reinterpret_cast<u32x2*>(rec + FREC_A + lane * 8) = ainv_bf;
         if (q4 == 0) *reinterpret_cast<float*>(rec + FREC_BETA + 4 * r) = beta;
     } else {
+        bcast_last([&](auto from_last) {
+            auto kgT = [&](int kt) {
+                return __builtin_bit_cast(u32x2, ONE_PASS ? get_T(scr.kg, kt, lane) : tile_T(kg_tile(kt, from_last), eye));
+            };
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const u32x2 k0 = __builtin_bit_cast(u32x2, get_T(scr.kg, 2 * j, lane));
-            const u32x2 k1 = __builtin_bit_cast(u32x2, get_T(scr.kg, 2 * j + 1, lane));
-            *reinterpret_cast<u32x4*>(rec + REC_KG + j * 1024 + lane * 16) = u32x4{k0.x, k0.y, k1.x, k1.y};
-        }
-#pragma unroll
-        for (int vt = 0; vt < 8; ++vt)
-            put_F(scr.kb, vt, lane, pack4(elem(vp, 4 * vt) * beta, elem(vp, 4 * vt + 1) * beta,
-                                          elem(vp, 4 * vt + 2) * beta, elem(vp, 4 * vt + 3) * beta));
-        wave_lds_fence();
-#pragma unroll
-        for (int vt = 0; vt < 8; ++vt) {
-            const u32x2 ub = form_u(get_T(scr.kb, vt, lane), A_op);
-            *reinterpret_cast<u32x2*>(rec + REC_U + vt * 512 + lane * 8) = ub;
-            if (p.dbg_u) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int row = 4 * q4 + i;
-                    if (row < nvalid) {
-                        const int64_t o = ((sp.tok0 + t0 + row) * HV + hv) * DK + 16 * vt + r;
-                        p.dbg_u[o] = (uint16_t)(i == 0 ? ub.x : i == 1 ? (ub.x >> 16)
-                                                : i == 2 ? ub.y : (ub.y >> 16));
-                    }
-                }
-            }
-        }
+            for (int j = 0; j < 4; ++j) store_pair(REC_KG, j, kgT(2 * j), kgT(2 * j + 1));
+        });
     }
 
     // ---- optional reference-layout intermediates (kernels.py:125,153,178-184)
@@ -554,14 +601,14 @@ __device__ __forceinline__ void k1_compute(const Params& p, int hv, int c, const
 // are tokens (every chunk but a sequence's partial last one), so the
 // row-validity selects and the rows mid = 8, last = 15 are compile-time.
 // GB16: g is bf16 (else fp32).
-template <int K1M, bool FULL, bool GB16>
+template <int K1M, bool FULL, bool GB16, bool ONE_PASS>
 __device__ __forceinline__ void k1_chunk(const Params& p, int hv, int c, const SeqSpan& sp,
                                          const K1Scratch& scr, uint8_t* rec) {
     K1In<GB16, K1M == K1_BOTH> in;
     k1_load<K1M, FULL, GB16>(p, hv, c, sp, in);
     const float* biasp = k1_bias(p, hv);
     const float ea = k1_ea(p, hv);
-    k1_compute<K1M, FULL, GB16>(p, hv, c, sp, in, biasp, ea, scr, rec);
+    k1_compute<K1M, FULL, GB16, ONE_PASS>(p, hv, c, sp, in, biasp, ea, scr, rec);
 }
 
 }  // namespace
