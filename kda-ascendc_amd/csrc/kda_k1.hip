@@ -134,11 +134,14 @@ hipError_t launch(const Params& p, hipStream_t stream) {
 //     60.6 / 64.8, 9216 69.8 / 70.3, 10240 81.8 / 79.0;
 //   packed sequences: 2000 (H=16) 25.8 / 25.6, 4000 32.6 / 36.0, 8100 61.3 /
 //     67.6, 16400 115.8 / 119.1, 33000 228.4 / 229.7.
-// fp32 g holds too much for four waves and never gains.
+// fp32 g holds too much for four waves and never gains, nor does a range of a
+// longer forward (6000 to 9000 chunks beside stage 2's traffic: T=4096 H=48
+// 167.7 us a forward, 170.3 in one pass; T=4003 H=64 199.8 and 201.6).
 static bool forward_in_one_pass(const Params& p) {
     const int64_t chunks = k1_grid(p);
     if (!p.g_bf16 || chunks <= 3072) return false;
     if (p.cu_seqlens) return true;
+    if (p.T != p.tok_stride) return false;
     return p.T % BT == 0 ? chunks > 3840 && chunks <= 7168 : chunks <= 9216;
 }
 
