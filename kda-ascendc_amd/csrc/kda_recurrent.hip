@@ -16,12 +16,12 @@
 // decode step (README.md:503-505).  No rounding happens between tokens, so
 // with o in fp32 the kernel is also an on-GPU gold for the chunked path.
 //
-// Two kernels, which give the same bits.  recurrent_kernel: the decode step and
-// fixed-length calls of two or three tokens whose states fill the chip, where the
-// states' bytes bound the call; recurrent_rows_kernel, below: everything else, bound
-// by the latency of the tokens.
+// Two kernels, which give the same bits.  recurrent_kernel: the decode step, and
+// calls of few tokens over many states, where the states' bytes bound the call;
+// recurrent_rows_kernel, below: everything else, bound by the latency of the
+// tokens (whole_states has the line between them).
 //
-// recurrent_kernel: one work-group of 256 threads per (batch row, value head).
+// recurrent_kernel: one work-group of 256 threads per (batch row or sequence, value head).
 // Thread t = 32 * hw + j holds the 64 state elements at memory offsets
 // 1024 * i + 4 * t + c (i = 0..15, c = 0..3) of the head's 128 x 128 state,
 // so every state load and store is a 16-byte access and each wave
@@ -34,7 +34,7 @@
 //     over i in registers, then over the eight half-waves: lane pairs of a
 //     wave by a shuffle, the four waves through LDS.
 // The state lives in registers for the whole sequence (64 floats per
-// thread; 106 to 161 VGPRs in all), so three or four work-groups share a CU and the
+// thread; 106 to 164 VGPRs in all), so three or four work-groups share a CU and the
 // decode step streams the states at close to the memory system's rate.
 // Grouped value heads (GVA): value head hv reads q/k head hv / (HV / H)
 // (kernels.py:88).  Varlen: the work-groups of a (sequence, value head) go over
@@ -153,7 +153,7 @@ __device__ __forceinline__ void store_o(const Params& p, int64_t idx, float x) {
 template <bool VFIRST, bool ONE>
 __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(ONE ? 4 : 1))) void recurrent_kernel(Params p) {
     const int HV = p.HV, H = p.H;
-    const int bhv = blockIdx.x;  // batch row * HV + hv
+    const int bhv = blockIdx.x;  // (batch row or sequence) * HV + hv
     const int hv = bhv - (bhv / HV) * HV;
     const int h = hv / (HV / H);
     const SeqSpan sp = seq_span(p, bhv);
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(ONE ? 4 : 1)
 // with the chip full, 2048 (sequence, head) pairs of 24 tokens: 232 -> 196 and
 // 316 -> 178.  Two waves a side instead of four: V-first 244 (the formers are
 // late); one former per work-group: 31 and 38 at the small size.
-// 107 VGPRs, 47 KB of LDS: two work-groups a CU.
+// 104 VGPRs and 48 KB of LDS V-first, 88 and 16 KB K-first: two work-groups a CU.
 //
 // The column groups and the order of the sums are recurrent_kernel's, so that
 // the two, and T decode steps and one call of T tokens, give the same bits:
@@ -597,22 +597,50 @@ __global__ __launch_bounds__(64 * (SW + SF)) void recurrent_rows_kernel(Params p
 
 }  // namespace
 
+// Whether recurrent_kernel takes a call of `tokens` tokens a pair, one token of
+// batch rows apart (that is always its).  Its three work-groups a CU hold 768
+// pairs at a time, with all of their states' bytes in flight; the two of
+// recurrent_rows_kernel hold 256, for a quarter to a third of the time a token.
+// So few tokens and full rounds are the former's.  Us, recurrent_kernel against
+// recurrent_rows_kernel (packed sequences; batch rows are within 3 % of them):
+//   V-first: 1 token, 256 pairs 10.4 / 8.6, 288 10.7 / 11.7, 768 18.4 / 24.7,
+//     4096 108 / 127; 2 tokens, 288 14.3 / 13.1, 384 15.2 / 15.9, 768 22.4 /
+//     26.9, 4096 120 / 139; 3 tokens, 640 25.4 / 25.6, 768 26.9 / 28.6, 960
+//     36.0 / 34.8, 2048 64.2 / 66.4, 4096 130 / 146; 4 tokens, 2560 98.3 /
+//     97.2, 3072 114 / 119; 5 tokens, 6144 241 / 241;
+//   K-first: 1 token, 256 9.5 / 8.5, 288 9.7 / 11.5, 4096 105 / 122; 2 tokens,
+//     768 20.4 / 24.0, 1792 46.8 / 44.2, 2048 51.7 / 54.8, 4096 120 / 122; 3
+//     tokens, 768 22.9 / 25.8, 1024 33.9 / 30.9; 5 tokens (the rows' second
+//     batch), 640 25.8 / 30.1, 1024 43.1 / 41.4, 2048 73.1 / 80.7, 8192 274 /
+//     320; 6 tokens, 640 29.3 / 30.4, 1024 47.6 / 42.2, 6144 228 / 238; 8
+//     tokens, 640 34.8 / 31.3, 768 35.8 / 36.8.
+static bool whole_states(bool v_first, int64_t pairs, int64_t tokens) {
+    constexpr int64_t ROUND = 768;
+    if (pairs <= 256 || tokens > 8) return false;
+    if (tokens <= 2) return tokens == 1 || pairs > 320;
+    const bool thin = pairs > ROUND && pairs <= 1024;  // a second round with little in it
+    if (v_first) return tokens == 3 ? pairs > 640 && !thin : tokens == 4 && pairs > 2816;
+    if (pairs <= ROUND) return pairs > (tokens == 5 ? 512 : tokens <= 6 ? 576 : 672);
+    return tokens == 5 ? !thin : tokens == 6 && pairs > 4096;
+}
+
 hipError_t launch_recurrent(const Params& p, hipStream_t stream) {
-    const int64_t pairs = (int64_t)(p.cu_seqlens ? p.N : p.B) * p.HV;
-    // Two or three tokens with the chip full spend their time on the states, of
-    // which recurrent_kernel has three work-groups' 64 KB a CU in flight where
-    // recurrent_rows_kernel has two of 32: V-first, 4096 pairs, 123 us against 139 at two
-    // tokens; 2048 pairs, 103 against 84 at six.  K-first the two are equal at
-    // two tokens (125 us), and up to 512 pairs (one round) V-first ones are.
-    const bool few = !p.cu_seqlens && p.T <= 3 && p.h0_v_first && pairs > 512;
+    const int64_t nseq = p.cu_seqlens ? p.N : p.B;
+    const int64_t pairs = nseq * p.HV;
+    // Packed sequences' lengths are on the device.  Where the tokens are a
+    // multiple of the sequences they are taken as equal, as a decode step's or
+    // a draft's are; else there may be a long one among them, for which
+    // recurrent_kernel takes up to four times as long a token.
+    const bool equal = !p.cu_seqlens || p.T % p.N == 0;
+    const int64_t tokens = p.cu_seqlens ? p.T / p.N : p.T;
     const bool one = !p.cu_seqlens && p.T == 1;
-    if (!one && !few) {
+    if (!one && !(equal && whole_states(p.h0_v_first, pairs, tokens))) {
         auto rows = p.h0_v_first ? recurrent_rows_kernel<true> : recurrent_rows_kernel<false>;
         hipLaunchKernelGGL(rows, dim3((unsigned)(pairs * SPLIT)), dim3(64 * (SW + SF)), 0, stream, p);
         return hipGetLastError();
     }
     auto kern = p.h0_v_first ? (one ? recurrent_kernel<true, true> : recurrent_kernel<true, false>)
-                             : recurrent_kernel<false, true>;
+                             : (one ? recurrent_kernel<false, true> : recurrent_kernel<false, false>);
     hipLaunchKernelGGL(kern, dim3((unsigned)pairs), dim3(RT), 0, stream, p);
     return hipGetLastError();
 }
