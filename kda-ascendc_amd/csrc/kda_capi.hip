@@ -179,7 +179,9 @@ int scratch_ptr(uint8_t** out) {
 int to_params_recurrent(const KdaBt16Args* a, Params& p) {
     int rc = check_common(a, p);
     if (rc != KDA_BT16_OK) return rc;
-    if (sequences(a) * a->HV > I32_MAX) return KDA_BT16_EUNSUPPORTED;
+    // (recurrent_kernel: 256 threads a pair in the grid's one dimension of at
+    // most 2^32 - 1)
+    if (sequences(a) * a->HV > 0xffffffffLL / 256) return KDA_BT16_EUNSUPPORTED;
     if (!a->q || !a->k || !a->v || !a->g || !a->beta || !a->o) return KDA_BT16_EINVAL;
     if (p.use_gate && !a->A_log) return KDA_BT16_EINVAL;
     if (a->dbg_Aqk || a->dbg_A_inv || a->dbg_w || a->dbg_u || a->dbg_g) return KDA_BT16_EINVAL;

@@ -477,8 +477,8 @@ __global__ __launch_bounds__(64 * (SW + SF)) void recurrent_rows_kernel(Params p
     const int bhv = blockIdx.x / SPLIT;  // (batch row or sequence) * HV + hv
     const int hv = bhv - (bhv / HV) * HV;
     const SeqSpan sp = seq_span(p, bhv);
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int len = sp.len;
 
     // The vectors of two times SF tokens: decay, k^, q^, each as four groups of
@@ -636,7 +636,9 @@ hipError_t launch_recurrent(const Params& p, hipStream_t stream) {
     const bool one = !p.cu_seqlens && p.T == 1;
     if (!one && !(equal && whole_states(p.h0_v_first, pairs, tokens))) {
         auto rows = p.h0_v_first ? recurrent_rows_kernel<true> : recurrent_rows_kernel<false>;
-        hipLaunchKernelGGL(rows, dim3((unsigned)(pairs * SPLIT)), dim3(64 * (SW + SF)), 0, stream, p);
+        // (a wave a row of the block: a dimension holds at most 2^32 - 1 threads,
+        // 8.4 M work-groups of 512 in one, which empty sequences reach)
+        hipLaunchKernelGGL(rows, dim3((unsigned)(pairs * SPLIT)), dim3(64, SW + SF), 0, stream, p);
         return hipGetLastError();
     }
     auto kern = p.h0_v_first ? (one ? recurrent_kernel<true, true> : recurrent_kernel<true, false>)
