@@ -303,8 +303,8 @@ __device__ __forceinline__ int fused_pair(const Params& p, int wg) {
 // One work-group per (sequence or batch row, value head).
 template <bool GB16>
 __global__ __launch_bounds__(F_THREADS) void fused_kernel(Params p) {
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int bh = fused_pair(p, blockIdx.x);
     const int hv = bh - (bh / p.HV) * p.HV;
     const SeqSpan sp = seq_span(p, bh);
@@ -324,15 +324,16 @@ __global__ __launch_bounds__(F_THREADS) void fused_kernel(Params p) {
         }
         __builtin_amdgcn_endpgm();
     }
-    if (threadIdx.x < F_RING) {
-        f_full[threadIdx.x] = 0;
-        f_done[threadIdx.x] = 0;
+    const int tid = 64 * wave + lane;
+    if (tid < F_RING) {
+        f_full[tid] = 0;
+        f_done[tid] = 0;
     }
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         f_aborted = 0;
         f_counted = 0;
     }
-    if (threadIdx.x < DK) f_bias[threadIdx.x] = p.use_gate && p.dt_bias ? p.dt_bias[hv * DK + threadIdx.x] : 0.f;
+    if (tid < DK) f_bias[tid] = p.use_gate && p.dt_bias ? p.dt_bias[hv * DK + tid] : 0.f;
     __syncthreads();
 
     if (wave >= F_NCW) {
@@ -434,7 +435,9 @@ bool fused_forward(const Params& p, int ncu) {
 hipError_t launch_fused(const Params& p, hipStream_t stream) {
     const int64_t nbh = (int64_t)(p.cu_seqlens ? p.N : p.B) * p.HV;
     auto kern = p.g_bf16 ? fused_kernel<true> : fused_kernel<false>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)nbh), dim3(F_THREADS), 0, stream, p);
+    // (a wave a row of the block: a dimension holds at most 2^32 - 1 threads, 5.6
+    // M work-groups of 768 in one, which short or empty sequences reach)
+    hipLaunchKernelGGL(kern, dim3((unsigned)nbh), dim3(64, F_NCW + F_NP), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -7,7 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from kda_bt16 import kda_recurrent_fwd
+from kda_bt16 import kda_bt16_fwd, kda_recurrent_fwd
 
 pytestmark = pytest.mark.gpu
 
@@ -34,5 +34,14 @@ def test_recurrence_over_more_than_2_pow_22_sequences(vfirst, gpu_device):
     x, cu, few, kw = _packed((1 << 22) + 4096, gpu_device)
     o, _ = kda_recurrent_fwd(*x, cu_seqlens=cu, state_v_first=vfirst, **kw)
     want, _ = kda_recurrent_fwd(*x, cu_seqlens=few, state_v_first=vfirst, **kw)
+    assert torch.isfinite(want).all()
+    assert torch.equal(o, want)
+
+
+def test_fused_forward_over_more_sequences_than_2_pow_32_threads(gpu_device):
+    # one work-group of 768 threads a sequence
+    x, cu, few, kw = _packed((1 << 32) // 768 + 4096, gpu_device)
+    o, _ = kda_bt16_fwd(*x, cu_seqlens=cu, use_fused_kernel=True, **kw)
+    want, _ = kda_bt16_fwd(*x, cu_seqlens=few, use_fused_kernel=True, **kw)
     assert torch.isfinite(want).all()
     assert torch.equal(o, want)
