@@ -20,8 +20,8 @@
 // alone are a sixth of it).  Twelve waves, three to a SIMD, so that two
 // others issue while one waits: with four producers at two waves per SIMD
 // the same work took as long as the waits it could not cover (B=16 T=2048
-// H=32: 490 us, and 450 us as it is now; 16 packed sequences in 8192 tokens,
-// 173 and 150 us).  The 168 registers of three waves per SIMD are the tight
+// H=32: 490 us, and 460 us as it is now; 16 packed sequences in 8192 tokens,
+// 173 and 151 us).  The 168 registers of three waves per SIMD are the tight
 // side: a few spilled registers in the compute waves' loop cost 30 %.
 // The arithmetic is stage 1's and the wide stage 2's, so o and ht are bit
 // for bit those of the two-stage forward.
@@ -164,8 +164,8 @@ __device__ __forceinline__ i32x4 buffer_words(const void* base, uint32_t bytes) 
 // One direct buffer->LDS load of 16 bytes a lane (lane l's to LDS address
 // lds + 16 l).  Written as inline asm so that the compiler, which cannot
 // tell which LDS bytes such a load writes, does not wait for it before every
-// later LDS access of the wave; the producer waits for it itself (vmcnt)
-// before it reads the staging area.  The load takes its LDS address from
+// later LDS access of the wave; the producer waits for it itself (vmcnt, in
+// tail()) before it marks the slot full.  The load takes its LDS address from
 // M0, which the block saves and restores (the compiler may hold a value
 // there); a wait state separates each M0 write from the next use, as the
 // compiler's own direct loads have.
@@ -338,9 +338,9 @@ __global__ __launch_bounds__(F_THREADS) void fused_kernel(Params p) {
 
     if (wave >= F_NCW) {
         // On the SIMD a producer shares with a compute wave it issues first:
-        // one long batch runs the same either way (B=16 T=2048 H=32: 450 us),
-        // 16 packed sequences in 8192 tokens in 150 us against 158 with the
-        // compute waves first or neither.
+        // one long batch runs the same either way (B=16 T=2048 H=32), 16 packed
+        // sequences in 8192 tokens in 150 us against 158 with the compute waves
+        // first or neither.
         __builtin_amdgcn_s_setprio(1);
         producer_wave<GB16>(p, wave - F_NCW, hv, sp);
         __builtin_amdgcn_endpgm();
@@ -383,15 +383,16 @@ __global__ __launch_bounds__(F_THREADS) void fused_kernel(Params p) {
 
 // Estimated times (us) of a varlen forward on `ncu` CUs, from per-chunk
 // costs measured on MI355X (K = V = 128, every in-kernel flag):
-//   fused: each work-group takes ~1.85 us per chunk of its sequence (1.74
-//   since it has eight producers; the line was measured at 1.85), in
+//   fused: each work-group takes ~1.85 us per chunk of its sequence, in
 //     parallel with the others, so the longest sequence sets the time, or
-//     the chunks per CU once the work-groups run in rounds;
+//     the chunks per CU once the work-groups run in rounds.  (Measured with
+//     four producers; with eight 1.55 to 1.8, so near the line the two
+//     stages are taken up to 15 % longer than the fused kernel would run.)
 //   two stages: stage 1 ~7.5 ns per record slot and value head, stage 2
 //     ~0.65 us per step of its longest chain (or of the chunks per CU).
-// Measured at 192 (sequence, head) pairs (HV = 32): lengths 19456 + 5 x
-// 1024, fused 2188 us and two stages 1146 (estimates 2250 and 1160);
-// 6 x 4096, 480 against 590 (474 and 536).
+// Measured at 256 (sequence, head) pairs (HV = 32): lengths 16384 + 7 x
+// 1024, fused 1580 us and two stages 1019 (estimates 1894 and 1021); 8 x
+// 2944, 329 against 544 (340 and 475).
 double fused_estimate_us(const Params& p, int ncu) {
     const double chunks = (double)((std::min(p.max_seqlen, p.T) + BT - 1) / BT);
     const double per_cu = (double)p.HV * p.NS / ncu;
@@ -413,14 +414,13 @@ double two_stage_estimate_us(const Params& p, int ncu) {
 // when the pairs fill the CUs.
 //
 // Below the CU count the fused kernel runs every pair in one round of
-// work-groups, about 1.74 us per chunk whatever their number, while the two
-// stages grow with the pairs (T=4096 forwards, two stages against fused: 128
-// pairs 377 against 476 us, 160 pairs 505 against 480, 224 pairs 658 against
-// 479).  With cu_seqlens the fused kernel's time follows the longest
-// sequence and stage 1's the total: a single long sequence among short ones
-// makes the fused kernel up to about twice slower (192 pairs, lengths
-// 19456 + 5 x 1024: fused 2188 us, two stages 1146; equal lengths: 480
-// against 590).  Without the length of the longest sequence, the pairs
+// work-groups, about 1.6 us per chunk whatever their number, while the two
+// stages grow with the pairs (T=4096 forwards, two stages against fused: 80
+// pairs 270 against 407 us, 128 pairs 371 against 406, 160 pairs 504 against
+// 409, 224 pairs 663 against 420).  With cu_seqlens the fused kernel's time
+// follows the longest sequence and stage 1's the total: a single long
+// sequence among short ones makes the fused kernel up to about twice slower
+// (the figures above).  Without the length of the longest sequence, the pairs
 // must fill the CUs.
 bool fused_forward(const Params& p, int ncu) {
     if (p.dbg_w || p.dbg_u || p.dbg_Aqk || p.dbg_A_inv || p.dbg_g) return false;

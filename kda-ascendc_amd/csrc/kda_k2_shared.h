@@ -42,7 +42,7 @@ __device__ __forceinline__ int longest_first(const Params& p, int s) {
 // 129 against 90.  Where all work-groups start at once their order does not
 // matter, and finding it costs a load and ~1 us.)  False past the last head
 // (grid: k2_grid).
-constexpr int CU_COUNT = 256;
+constexpr int CU_COUNT = 256;  // of a whole card; on fewer the order only differs for the sizes in between
 template <int NSL>
 __device__ __forceinline__ bool k2_pair(const Params& p, int wg, int& bh, int& slice) {
     const int nbh = (p.cu_seqlens ? p.N : p.B) * p.HV;

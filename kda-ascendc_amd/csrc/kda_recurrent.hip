@@ -135,9 +135,6 @@ __device__ __forceinline__ void load_tok(const Params& p, const SeqSpan& sp, int
     r.beta = load_scalar(p.beta, p.beta_bf16, rv);
 }
 
-__device__ __forceinline__ float lo16(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
-__device__ __forceinline__ float hi16(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
-
 __device__ __forceinline__ void store_o(const Params& p, int64_t idx, float x) {
     if (p.o_fp32) {
         reinterpret_cast<float*>(p.o)[idx] = x;
@@ -201,8 +198,8 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(ONE ? 4 : 1)
 
         if constexpr (VFIRST) {
             // this thread's columns of q^, k^ and the decay
-            float qv[4] = {lo16(cur.q.x), hi16(cur.q.x), lo16(cur.q.y), hi16(cur.q.y)};
-            float kv[4] = {lo16(cur.k.x), hi16(cur.k.x), lo16(cur.k.y), hi16(cur.k.y)};
+            float qv[4] = {lo_f(cur.q.x), hi_f(cur.q.x), lo_f(cur.q.y), hi_f(cur.q.y)};
+            float kv[4] = {lo_f(cur.k.x), hi_f(cur.k.x), lo_f(cur.k.y), hi_f(cur.k.y)};
             if (p.use_l2norm) {
                 float sq = 0.f, sk = 0.f;
 #pragma unroll
@@ -224,7 +221,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(ONE ? 4 : 1)
             float* sv = s_v[tt & 1];
             if (vlane)
                 *reinterpret_cast<f32x4*>(sv + 4 * t) =
-                    f32x4{lo16(cur.v.x), hi16(cur.v.x), lo16(cur.v.y), hi16(cur.v.y)};
+                    f32x4{lo_f(cur.v.x), hi_f(cur.v.x), lo_f(cur.v.y), hi_f(cur.v.y)};
             __syncthreads();
             float ov = 0.f;  // o of row 8 * j + hw, kept by lane j < 16
 #pragma unroll
@@ -250,8 +247,8 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(ONE ? 4 : 1)
         } else {
             // wave 0 forms the token's decay, k^ and q^ for the work-group
             if (w == 0) {
-                float q0 = lo16(cur.q.x), q1 = hi16(cur.q.x);
-                float k0 = lo16(cur.k.x), k1 = hi16(cur.k.x);
+                float q0 = lo_f(cur.q.x), q1 = hi_f(cur.q.x);
+                float k0 = lo_f(cur.k.x), k1 = hi_f(cur.k.x);
                 if (p.use_l2norm) {
                     float sq = fmaf(q0, q0, q1 * q1), sk = fmaf(k0, k0, k1 * k1);
                     sq = half_sum(sq);
@@ -292,7 +289,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(ONE ? 4 : 1)
             if ((t & 32) == 0)
                 *reinterpret_cast<f32x4*>(&s_red[0][w][4 * j]) = f32x4{part[0], part[1], part[2], part[3]};
             __syncthreads();
-            const float vv[4] = {lo16(cur.v.x), hi16(cur.v.x), lo16(cur.v.y), hi16(cur.v.y)};
+            const float vv[4] = {lo_f(cur.v.x), hi_f(cur.v.x), lo_f(cur.v.y), hi_f(cur.v.y)};
             float vnew[4];
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
@@ -417,11 +414,10 @@ struct FormRaw {
     uint16_t v;  // row v0 + lane
 };
 
-template <bool VFIRST>
 __device__ __forceinline__ f32x2 load_g2(const Params& p, int64_t at) {
     if (p.g_bf16) {
         const uint32_t w = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(p.g) + at);
-        return f32x2{lo16(w), hi16(w)};
+        return f32x2{lo_f(w), hi_f(w)};
     }
     return *reinterpret_cast<const f32x2*>(static_cast<const float*>(p.g) + at);
 }
@@ -438,9 +434,9 @@ __device__ __forceinline__ void load_form(const Params& p, const SeqSpan& sp, in
         r.q.x = *reinterpret_cast<const uint32_t*>(p.q + rq * DK + col);
         r.k.x = *reinterpret_cast<const uint32_t*>(p.k + rq * DK + col);
     }
-    r.g = load_g2<VFIRST>(p, rv * DK + col);
+    r.g = load_g2(p, rv * DK + col);
     r.gp = f32x2{0.f, 0.f};
-    if (!p.use_gate && !p.g_log && tt % BT != 0) r.gp = load_g2<VFIRST>(p, (rv - p.HV) * DK + col);
+    if (!p.use_gate && !p.g_log && tt % BT != 0) r.gp = load_g2(p, (rv - p.HV) * DK + col);
     r.beta = load_scalar(p.beta, p.beta_bf16, rv);
     r.v = p.v[rv * DK + v0 + lane];
 }
@@ -451,14 +447,14 @@ __device__ __forceinline__ f32x2 unit2(const Params& p, u32x2 w, int lane) {
     f32x2 y;
     if constexpr (VFIRST) {
         const uint32_t mine = lane < 32 ? w.x : w.y;
-        y = f32x2{lo16(mine), hi16(mine)};
+        y = f32x2{lo_f(mine), hi_f(mine)};
     } else {
-        y = f32x2{lo16(w.x), hi16(w.x)};
+        y = f32x2{lo_f(w.x), hi_f(w.x)};
     }
     if (!p.use_l2norm) return y;
     float ss;
     if constexpr (VFIRST) {
-        const float c[4] = {lo16(w.x), hi16(w.x), lo16(w.y), hi16(w.y)};
+        const float c[4] = {lo_f(w.x), hi_f(w.x), lo_f(w.y), hi_f(w.y)};
         ss = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) ss = fmaf(c[i], c[i], ss);
