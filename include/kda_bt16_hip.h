@@ -260,7 +260,8 @@ int kda_bt16_k2_hip(const KdaBt16Args* args, void* stream);
  *   - o is fp32 with KDA_BT16_O_FP32, else bf16;
  *   - no workspace and no debug outputs (workspace fields are ignored, the
  *     debug pointers must be NULL);
- *   - h0 and ht may be the same buffer (the state updated in place). */
+ *   - h0 and ht may be the same buffer (the state updated in place);
+ *   - at most 2^24 - 1 (row or sequence, value head) pairs. */
 int kda_recurrent_fwd_hip(const KdaBt16Args* args, void* stream);
 
 /* Backward of the chunked forward (no counterpart in the reference, which is

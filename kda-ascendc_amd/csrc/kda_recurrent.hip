@@ -342,9 +342,9 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(ONE ? 4 : 1)
 // Bound by the latency of a token's chain (LDS reads, 32 products, the exchange,
 // the update, 32 products), 0.75 us a token where recurrent_kernel's reductions
 // across lanes (V-first) or waves (K-first) take 2.1 (K-first) to 3.1 (V-first).
-// Four sequences of 24 tokens at 16 heads: 57 -> 26 us K-first, 81 -> 25 V-first;
-// with the chip full, 2048 (sequence, head) pairs of 24 tokens: 232 -> 196 and
-// 316 -> 178.  Two waves a side instead of four: V-first 244 (the formers are
+// Four sequences of 24 tokens at 16 heads: 55 -> 21 us K-first, 77 -> 19 V-first;
+// with the chip full, 2048 (sequence, head) pairs of 24 tokens: 221 -> 191 and
+// 308 -> 179.  Two waves a side instead of four: V-first 244 (the formers are
 // late); one former per work-group: 31 and 38 at the small size.
 // 104 VGPRs and 48 KB of LDS V-first, 88 and 16 KB K-first: two work-groups a CU.
 //
